@@ -11,7 +11,8 @@ struct DensePlan {
     void *afrag;        // [A0 | A1] in MFMA A-fragment order
     void *arow;         // [A0 | A1] row-major (scalar kernel)
     int variant;        // 0: scalar kernel; 1, 2, 4: MFMA, wavefronts per
-                        // block; 16 + (1, 2, 4): operator staged in LDS
+                        // block; 16 + (1, 2, 4): operator staged in LDS;
+                        // + 256 s: row tiles split over s row groups
 };
 
 // BF16-operand plans (FP32 data and accumulation): k steps of 16

@@ -172,6 +172,14 @@ __device__ __forceinline__ void epi1(T acc, T *__restrict__ c, long off,
 }
 
 // ---- MFMA kernel ----------------------------------------------------------
+//
+// One wavefront per 64 columns and group of MT row tiles (blockIdx.y).  An
+// operator of more than 7 tiles (112 rows: the gradient operators of prisms
+// and pyramids from p = 3, anti-aliased hex operators) does not fit one
+// wavefront's accumulators and is split; so is a shorter one where there
+// are too few 64-column groups to fill the chip (the tuner decides).  Each
+// group reads B again, from the L2.  Before, operators past 7 tiles ran on
+// the scalar kernel: 120 x 40 on 726 FP64 prisms took 905 us, now 19 us.
 template <typename T, int MT, int EP>
 __device__ __forceinline__ void dense_tiles(
     int m, int ks0, int ks1, int k0, int k1, const T *__restrict__ af,
@@ -186,6 +194,7 @@ __device__ __forceinline__ void dense_tiles(
     const int kr = lane >> 4, cq = (lane & 15)*4;
     const int KS = ks0 + ks1;
     const int W = blockDim.x >> 6;
+    const int mt0 = blockIdx.y*MT;       // this row group's first tile
     const T *afl = af + lane;
     {
     const long g = (long)blockIdx.x*W + (threadIdx.x >> 6);
@@ -241,7 +250,8 @@ __device__ __forceinline__ void dense_tiles(
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const int row = 16*mt + (sizeof(T) == 8 ? kr + 4*r : 4*kr + r);
+            const int row = 16*(mt0 + mt) +
+                            (sizeof(T) == 8 ? kr + 4*r : 4*kr + r);
             if (row >= m) continue;
             const long off = row*ldc + c0 + cq;
             if constexpr (EP == 0) {
@@ -290,7 +300,9 @@ __global__ __launch_bounds__(256) void k_dense_mfma(
     long ldr, int nvar, void *__restrict__ xa, double dta, double dtb,
     T alpha, T beta)
 {
-    const T *a = LDSA ? stage_frags(af, MT*(ks0 + ks1)*64) : af;
+    const long nf = (long)MT*(ks0 + ks1)*64;
+    af += blockIdx.y*nf;
+    const T *a = LDSA ? stage_frags(af, (int)nf) : af;
     dense_tiles<T, MT, EP>(m, ks0, ks1, k0, k1, a, ncol, b0, ld0, b1, ld1, c,
                            ldc, rcp, ldr, nvar, xa, dta, dtb, alpha, beta);
 }
@@ -814,7 +826,8 @@ __attribute__((amdgpu_waves_per_eu(G <= 10 ? 4 : 2))) void k_tdivf_flux4(
 
 // Variant codes: 0 scalar kernel; 1, 2, 4 MFMA with that many wavefronts
 // per block and the operator read through the L2; 16 + (1, 2, 4) the same
-// with the operator staged in LDS once per block.
+// with the operator staged in LDS once per block; + 256 s: the operator's
+// row tiles split over s row groups (s = 0: as few as fit).
 constexpr int FR_LDSV = 16;
 // flux-fused kernels only: the block-cooperative form (five wavefronts per
 // element block, flux evaluated once into LDS)
@@ -827,12 +840,35 @@ constexpr int FR_V4 = 64;
 constexpr int FR_V4B = 65;
 constexpr size_t FR_LDS_MAX = 65536;
 
+// Row tiles one wavefront's accumulators hold
+constexpr int FR_MTMAX = 7;
+constexpr int FR_SPLIT = 256;
+
+// Row tiles per group of an operator of mt tiles under variant v
+static int group_tiles(int v, int mt)
+{
+    const int least = (mt + FR_MTMAX - 1)/FR_MTMAX;
+    const int s = std::max(v/FR_SPLIT, least);
+    return (mt + s - 1)/s;
+}
+
 static bool variant_valid(int v, size_t ldsbytes, bool scalar_ok)
 {
     const int w = v & ~FR_LDSV;
     if (v == 0) return scalar_ok;
     if (w != 1 && w != 2 && w != 4) return false;
     return !(v & FR_LDSV) || ldsbytes <= FR_LDS_MAX;
+}
+
+// The same for dense plans, whose variants also split the row tiles
+static bool dense_valid(const DensePlan *p, int v)
+{
+    if (v < 0 || v/FR_SPLIT > p->mt) return false;
+    const size_t esz = p->dtype == FRHIP_F64 ? 8 : 4;
+    const int b = v % FR_SPLIT;
+    if (b == 0 && v) return false;
+    return variant_valid(b, (size_t)group_tiles(v, p->mt)*(p->ks0 + p->ks1)*
+                                64*esz, true);
 }
 
 template <typename T, int EP>
@@ -852,27 +888,27 @@ static int launch_ep(const DensePlan *p, int variant, long ncol,
                            (T)alpha, (T)beta);
         return 0;
     }
-    const int wpb = variant & ~FR_LDSV;      // wavefronts per block
+    const int mtg = group_tiles(variant, p->mt);   // tiles per row group
+    const int wpb = variant % FR_SPLIT & ~FR_LDSV; // wavefronts per block
     const bool lds = variant & FR_LDSV;
-    const size_t ldsb = lds ? (size_t)p->mt*(p->ks0 + p->ks1)*64*sizeof(T)
-                            : 0;
+    const size_t ldsb = lds ? (size_t)mtg*(p->ks0 + p->ks1)*64*sizeof(T) : 0;
     dim3 block(64*wpb);
 #define FR_MT(MTV)                                                          \
     case MTV: {                                                             \
         auto k = lds ? k_dense_mfma<T, MTV, EP, true>                       \
                      : k_dense_mfma<T, MTV, EP, false>;                     \
-        dim3 grid(cdiv(ncol/64, wpb));                                      \
+        dim3 grid(cdiv(ncol/64, wpb), cdiv(p->mt, MTV));                    \
         hipLaunchKernelGGL(k, grid, block, ldsb, s, p->m, p->ks0, p->ks1,   \
                            p->k0, p->k1, (const T *)p->afrag, ncol, pb0,    \
                            ld0, pb1, ld1, (T *)c, ldc, prcp, ldr, nvar, xa, \
                            dta, dtb, (T)alpha, (T)beta);                    \
         return 0;                                                           \
     }
-    switch (p->mt) {
+    switch (mtg) {
         FR_MT(1) FR_MT(2) FR_MT(3) FR_MT(4) FR_MT(5) FR_MT(6) FR_MT(7)
     }
 #undef FR_MT
-    set_error("dense operator too tall for the MFMA kernel");
+    set_error("invalid dense row split");
     return 2;
 }
 
@@ -914,7 +950,7 @@ static bool mfma_ok(const DensePlan *p, long ncol, const void *b0, long ld0,
     auto al = [va](const void *q) {
         return q == nullptr || (reinterpret_cast<uintptr_t>(q) % va) == 0;
     };
-    return p->mt >= 1 && p->mt <= 7 && ncol % 64 == 0 && ld0 % 4 == 0 &&
+    return ncol % 64 == 0 && ld0 % 4 == 0 &&
            (p->k1 == 0 || ld1 % 4 == 0) && ldc % 4 == 0 && al(b0) &&
            al(b1) && al(c);
 }
@@ -931,7 +967,8 @@ int dense_plan_create(DensePlan **out, int m, int k0, int k1,
         return q < k0 ? a0[(long)r*k0 + q] : a1[(long)r*k1 + q - k0];
     };
 
-    std::vector<double> frag((size_t)mt*KS*64, 0.0);
+    // the last row group of a split may run past the operator: zero tiles
+    std::vector<double> frag((size_t)(mt + FR_MTMAX - 1)*KS*64, 0.0);
     for (int t = 0; t < mt; ++t)
         for (int s = 0; s < KS; ++s)
             for (int l = 0; l < 64; ++l) {
@@ -963,7 +1000,7 @@ int dense_plan_create(DensePlan **out, int m, int k0, int k1,
     };
 
     DensePlan *p = new DensePlan{m, k0, k1, dtype, mt, ks0, ks1, nullptr,
-                                 nullptr, mt <= 7 ? 4 : 0};
+                                 nullptr, 4};
     if (upload(frag, &p->afrag) || upload(row, &p->arow)) {
         dense_plan_destroy(p);
         return 1;
@@ -974,9 +1011,7 @@ int dense_plan_create(DensePlan **out, int m, int k0, int k1,
 
 bool dense_variant_ok(const DensePlan *p, int variant)
 {
-    const size_t esz = p->dtype == FRHIP_F64 ? 8 : 4;
-    return variant_valid(variant, (size_t)p->mt*(p->ks0 + p->ks1)*64*esz,
-                         true);
+    return dense_valid(p, variant);
 }
 
 void dense_plan_destroy(DensePlan *p)
@@ -995,10 +1030,19 @@ int dense_launch(const DensePlan *p, int ep, long ncol, const void *b0,
     int variant = p->variant;
     if (variant != 0 && !mfma_ok(p, ncol, b0, ld0, b1, ld1, c, ldc))
         variant = 0;
-    const size_t esz = p->dtype == FRHIP_F64 ? 8 : 4;
-    if (!variant_valid(variant, (size_t)p->mt*(p->ks0 + p->ks1)*64*esz,
-                       true))
+    if (!dense_valid(p, variant))
         variant &= ~FR_LDSV;
+    // in place, each column's reads of B must precede its writes: one
+    // wavefront for all rows
+    const size_t esz = p->dtype == FRHIP_F64 ? 8 : 4;
+    auto meets = [&](const void *b, int k, long ld) {
+        const uintptr_t b0p = (uintptr_t)b, cp = (uintptr_t)c;
+        return b && b0p < cp + ((p->m - 1)*ldc + ncol)*esz &&
+               cp < b0p + ((k - 1)*ld + ncol)*esz;
+    };
+    if (variant >= FR_SPLIT && (meets(b0, p->k0, ld0) ||
+                                meets(p->k1 ? b1 : nullptr, p->k1, ld1)))
+        variant %= FR_SPLIT;
     const int rc = p->dtype == FRHIP_F64
         ? launch_t<double>(p, variant, ep, ncol, b0, ld0, b1, ld1, c, ldc,
                            rcp, ldr, nvar, xa, dta, dtb, alpha, beta, s)
@@ -1027,12 +1071,24 @@ int dense_tune(DensePlan *p, long ncol, const void *b0, long ld0,
     hipEvent_t e0, e1;
     (void)hipEventCreate(&e0);
     (void)hipEventCreate(&e1);
-    const int cands[] = {0, 1, 2, 4, FR_LDSV + 1, FR_LDSV + 2, FR_LDSV + 4};
-    const size_t ldsb = (size_t)p->mt*(p->ks0 + p->ks1)*64*esz;
+    // The scalar kernel never wins where the MFMA kernel runs (60 us against
+    // 4.5 at its closest, 30 rows on 4,374 FP32 tets).  Row groups beyond
+    // the fewest that fit pay only while the finer grid is still short of
+    // two wavefronts per SIMD (2,048 of them on the chip): each re-reads B.
+    std::vector<int> cands = {1, 2, 4, FR_LDSV + 1, FR_LDSV + 2,
+                              FR_LDSV + 4};
+    const int least = (p->mt + FR_MTMAX - 1)/FR_MTMAX;
+    for (int s = least + 1, last = group_tiles(0, p->mt); s <= p->mt; ++s) {
+        const int t = group_tiles(s*FR_SPLIT, p->mt);
+        if (t == last) continue;
+        last = t;
+        if (ncol/64*(s - 1) >= 2048) break;
+        for (int w : {1, 2, 4}) cands.push_back(s*FR_SPLIT + w);
+    }
     float best = 1e30f;
     int bestv = p->variant, rc = 0;
     for (int v : cands) {
-        if (!variant_valid(v, ldsb, true)) continue;
+        if (!dense_valid(p, v)) continue;
         DensePlan q = *p;
         q.variant = v;
         for (int it = 0; it < reps + 1 && !rc; ++it) {

@@ -105,6 +105,43 @@ def test_dense_variants_agree(backend_factory, precision, variant, shape):
 
 
 @pytest.mark.parametrize('precision', ['double', 'single'])
+@pytest.mark.parametrize('variant', [None, 4, 17, 2*256 + 1, 3*256 + 4])
+@pytest.mark.parametrize('shape', [(112, 20, 3), (113, 40, 5),
+                                   (225, 75, 105)])
+def test_dense_row_groups(backend_factory, precision, variant, shape):
+    """Operators at and past the rows one wavefront holds (7 tiles of 16):
+    the row groups the kernel splits them into, the last of them short,
+    with the tuner's choice (None) and forced splits."""
+    import ctypes as ct
+    from pyfr_amd._lib import FrHipError
+    be = backend_factory(precision=precision)
+    m, k0, k1 = shape
+    A0, A1, b0, b1, c, _ = _operands(be, m, k0, k1, 70, sum(shape))
+    p = _Plan2(be, A0, A1)
+    assert p.kind == 2
+    print(f'\n[row groups] {precision} {shape} v={variant}', flush=True)
+    if variant is None:
+        v = ct.c_int()
+        be.lib.mul2_plan_tune(p.plan, c.ncol, b0.data, b0.leaddim, b1.data,
+                              b1.leaddim, 2, ct.byref(v))
+        assert v.value > 0
+    else:
+        try:
+            be.lib.mul2_plan_set_variant(p.plan, variant)
+        except FrHipError:
+            # a row group's operator past the LDS budget
+            assert variant & 16
+            return
+    be.lib.mul2(p.plan, c.ncol, b0.data, b0.leaddim, b1.data, b1.leaddim,
+                c.data, c.leaddim, 0, None, 0, None, 0.0, 0.0, 0, be.stream)
+    be.wait()
+    ref = ((A0 @ b0.get().reshape(k0, -1) + A1 @ b1.get().reshape(k1, -1))
+           .reshape(m, 5, 70))
+    tol = 1e-13 if precision == 'double' else 2e-6
+    assert rel_l2(c.get(), ref) < tol
+
+
+@pytest.mark.parametrize('precision', ['double', 'single'])
 @pytest.mark.parametrize('per_element', [True, False])
 @pytest.mark.parametrize('ep,last', [(1, 0), (2, 0), (2, 1)])
 def test_dense_epilogues(backend_factory, precision, per_element, ep, last):
