@@ -163,6 +163,32 @@ int frhip_mul2_plan_tune(void *plan, int ncol, const void *b0, long ld0,
 int frhip_mul_plan_set_variant(void *plan, int variant);
 int frhip_mul2_plan_set_variant(void *plan, int variant);
 
+/* ---- element-local passes of hexes whose operators act along the lines of
+ *      Gauss-Legendre solution points (no counterpart in the reference: they
+ *      fuse the kernels named below) ----
+ * A plan holds the 1-D operators of n = p + 1 points (2..5): d (n x n, row
+ * major) the derivative corrected for the interior traces (the line block
+ * of M1 - M3*M2 and of M4 - M6*M0), hl / hr the correction functions of the
+ * low / high end, ll / lr the traces there, x the points. */
+int frhip_hex_plan_create(void **plan, int n, const double *d,
+                          const double *hl, const double *hr,
+                          const double *ll, const double *lr,
+                          const double *x, int dtype);
+int frhip_hex_plan_destroy(void *plan);
+/* geo = FRHIP_GEO_CURVED / FRHIP_GEO_HEX_LINEAR: tdisf (Euler, pyfr/solvers/
+ * euler/kernels/tflux.mako:8-30) + tdivtpcorf + tdivtconf + negdivconf of
+ * the solution u (n^3, 5, neles); gm: smats or vertices.  geo = -1: u holds
+ * the volume part of the transformed divergence (frhip_hex_nsvol) and
+ * tdivtconf + negdivconf are applied.  f (6 n^2, 5, neles): the common
+ * normal fluxes.  ep (1-3, 10-17), c, rcp (a value per point), xa, dta, dtb
+ * and last as for frhip_mul2.  disu (stages that form a next input): f
+ * receives M0 of that input.  c and xa may be u.  base: as frhip_tflux_euler. */
+int frhip_hex_div(void *plan, int geo, int neles, const void *u, long ldu,
+                  const void *gm, long ldg, void *f, long ldf, void *c,
+                  long ldc, int ep, const void *rcp, long ldr, void *xa,
+                  double dta, double dtb, int last, int disu, double gamma,
+                  const double *base, void *stream);
+
 /* ---- flux-fused divergence for straight-sided tets and prisms (Euler):
  *      tdisf (pyfr/solvers/euler/kernels/tflux.mako:8-30) + tdivtpcorf +
  *      tdivtconf + negdivconf (pyfr/solvers/baseadvec/elements.py:84-119)

@@ -60,6 +60,11 @@ _FUNCS = {
     'frhip_mul2_plan_set_variant': [_P, _I],
     'frhip_mul2': [_P, _I, _P, _L, _P, _L, _P, _L, _I, _P, _L, _P, _D, _D,
                    _I, _P],
+    'frhip_hex_plan_create': [ct.POINTER(_P), _I, _P, _P, _P, _P, _P, _P,
+                              _I],
+    'frhip_hex_plan_destroy': [_P],
+    'frhip_hex_div': [_P, _I, _I, _P, _L, _P, _L, _P, _L, _P, _L, _I, _P,
+                      _L, _P, _D, _D, _I, _I, _D, _P, _P],
     'frhip_tdivf_plan_create': [ct.POINTER(_P), _I, _I, _I, _P, _P, _I],
     'frhip_tdivf_plan_destroy': [_P],
     'frhip_tdivf_plan_tune': [_P, _I, _P, _L, _P, _L, _P, _L, _D, _I,

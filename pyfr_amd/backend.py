@@ -430,10 +430,16 @@ class Concurrent:
 
 
 def flat_kernels(items):
-    """The kernels of a list of kernels and Concurrent groups, in order."""
+    """The kernels of a list of kernels, meta kernels and Concurrent groups,
+    in order."""
     out = []
     for k in items:
-        out += k.kernels() if isinstance(k, Concurrent) else [k]
+        if isinstance(k, Concurrent):
+            out += flat_kernels(k.kernels())
+        elif isinstance(k, MetaKernel):
+            out += flat_kernels(k.kernels)
+        else:
+            out.append(k)
     return out
 
 
@@ -596,6 +602,20 @@ def _check_xa(xa, out, ep):
                              'shape, leading dimension and precision')
 
 
+def _ptr_triple(be, r1, r0):
+    """Device pointers {r1, r0, dt} for an RK4 epilogue, dt a device double
+    of its own (each kernel binds its step there).  Returns (address of the
+    pointer array, address of dt); both are tracked by the backend, which
+    frees them at teardown."""
+    dtp = be._malloc_impl(8)
+    be.lib.fill_f64(dtp, 1, 0.0, None)
+    h = np.array((r1.data, r0.data, dtp), dtype=np.uint64)
+    p = be._malloc_impl(h.nbytes)
+    be.lib.memcpy_htod(p, h.ctypes.data, h.nbytes, None)
+    be.lib.stream_sync(None)
+    return p, dtp
+
+
 class MulProvider:
     """``mul``: structured (sparsity-pattern matched) or dense operator
     kernels; replaces the GiMMiK/rocBLAS providers."""
@@ -701,7 +721,7 @@ class MulProvider:
         if ep >= 10:
             # RK4 stages: xa = (r1, r0), passed with the step's device
             # scalar as the device pointers {r1, r0, dt}
-            xap, dtp = self._ptr_triple(*xa)
+            xap, dtp = _ptr_triple(self.backend, *xa)
             xam = tuple(xa)
         else:
             xap, xam, dtp = None if xa is None else xa.data, (), None
@@ -799,7 +819,7 @@ class MulProvider:
         _check_xa(xa, out, ep)
         if ep >= 10:
             # RK4 stages: xa = (r1, r0) with the step's device scalar
-            xap, dtp = self._ptr_triple(*xa)
+            xap, dtp = _ptr_triple(self.backend, *xa)
         else:
             xap, dtp = None if xa is None else xa.data, None
         args = (plan, ncol, u.data, u.leaddim, smats.data, smats.leaddim,
@@ -820,20 +840,6 @@ class MulProvider:
         k.kind = 'dense'
         return k
 
-    def _ptr_triple(self, r1, r0):
-        """Device pointers {r1, r0, dt} for an RK4 epilogue, dt a device
-        double of its own (each kernel binds its step there).  Returns
-        (address of the pointer array, address of dt); both are tracked by
-        the backend, which frees them at teardown."""
-        be = self.backend
-        dtp = be._malloc_impl(8)
-        be.lib.fill_f64(dtp, 1, 0.0, None)
-        h = np.array((r1.data, r0.data, dtp), dtype=np.uint64)
-        p = be._malloc_impl(h.nbytes)
-        be.lib.memcpy_htod(p, h.ctypes.data, h.nbytes, None)
-        be.lib.stream_sync(None)
-        return p, dtp
-
     def __del__(self):
         try:
             for plan, _, _ in self._plans.values():
@@ -842,6 +848,77 @@ class MulProvider:
                 self.backend.lib.mul2_plan_destroy(plan)
             for plan, _, _ in self._plans3.values():
                 self.backend.lib.tdivf_plan_destroy(plan)
+        except Exception:
+            pass
+
+
+class HexLineProvider:
+    """Element-local passes of hexes whose operators act along lines
+    (``HexShape.lines``); no reference counterpart: they fuse kernels the
+    reference runs one after the other (see include/frhip.h)."""
+
+    def __init__(self, backend):
+        self.backend = backend
+        self._plans = {}
+
+    def _plan(self, basis, dtype):
+        if not getattr(basis, 'has_lines', False) or basis.n > 5:
+            raise NotSuitableError('needs line operators of at most 5 points')
+        key = (basis.n, dtype)
+        if key not in self._plans:
+            ops = [np.ascontiguousarray(m, dtype=np.float64)
+                   for m in basis.lines]
+            plan = ct.c_void_p()
+            self.backend.lib.hex_plan_create(
+                ct.byref(plan), basis.n, *[m.ctypes.data for m in ops],
+                _dtcode(dtype))
+            self._plans[key] = plan.value
+        return self._plans[key]
+
+    def hexdiv(self, basis, geo, neles, u, fn, out, rcpdjac, gamma=0.0,
+               metric=None, xa=None, stage=None, disu=False, base=None):
+        """[tdisf +] tdivtpcorf + tdivtconf + negdivconf (+ the stage update,
+        as ``MulProvider.tdivf``, + with disu the next stage's disu into
+        fn) over neles elements.  geo: the geometry mode of metric, or -1
+        where u is the volume divergence of ``hexnsvol``."""
+        ep = _STAGE_EP[stage]
+        nu, nf = basis.nupts, basis.nfpts
+        if (u.nrow < nu or fn.nrow != nf or out.nrow != nu or
+                any(m.ncol != out.ncol or m.dtype != out.dtype
+                    for m in (u, fn)) or rcpdjac.nrow != nu):
+            raise ValueError('Incompatible matrices for hexdiv')
+        plan = self._plan(basis, out.dtype)
+        if ep in (3, 14, 15, 16, 17) and out.dtype != np.float32:
+            raise NotSuitableError('the precision form needs FP32 operands')
+        _check_xa(xa, out, ep)
+        if ep >= 10:
+            xap, dtp = _ptr_triple(self.backend, *xa)
+        else:
+            xap, dtp = None if xa is None else xa.data, None
+        lib = self.backend.lib
+        bs = None if base is None else (ct.c_double*2)(*base)
+        args = (plan, geo, neles, u.data, u.leaddim,
+                None if metric is None else metric.data,
+                0 if metric is None else metric.leaddim, fn.data, fn.leaddim,
+                out.data, out.leaddim, ep, rcpdjac.data, rcpdjac.leaddim, xap)
+
+        def fn_(stream, dta=0.0, dtb=0.0, last=0):
+            lib.hex_div(*args, dta, dtb, int(last), int(disu), gamma, bs,
+                        stream)
+        rt = {'dtb': 0.0, 'last': 0}
+        if dtp is None:
+            rt['dta'] = 0.0
+        k = Kernel(fn_, rtargs=rt, mats=(u, fn, out, rcpdjac, metric),
+                   name=f'hexdiv{"" if geo >= 0 else "c"}_ep{ep}')
+        if dtp is not None:
+            k.devargs = {'dta': (dtp, self.backend)}
+        k.disu = disu
+        return k
+
+    def __del__(self):
+        try:
+            for plan in self._plans.values():
+                self.backend.lib.hex_plan_destroy(plan)
         except Exception:
             pass
 
@@ -1345,7 +1422,7 @@ class AMDBackend:
 
         self.pointwise = PointwiseProvider(self)
         self._providers = [self.pointwise, BlasExtProvider(self),
-                           MulProvider(self)]
+                           MulProvider(self), HexLineProvider(self)]
 
     # -- memory
     def _extent_alloc_bytes(self, nbytes):

@@ -14,6 +14,7 @@ BUILD = os.path.join(CSRC, '_build')
 LIB = os.path.join(HERE, 'libfrhip.so')
 
 SOURCES = ['frhip_runtime.hip', 'frhip_ops.hip', 'frhip_dense.hip',
+           'frhip_hex.hip',
            'frhip_pointwise.hip', 'frhip_bcs.hip', 'frhip_blasext.hip']
 
 HIPFLAGS = [

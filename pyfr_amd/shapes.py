@@ -313,6 +313,23 @@ class HexShape:
     def hend(self):
         return {s: legendre_kernel_end(self.x1d, s) for s in (-1, +1)}
 
+    @property
+    def has_lines(self):
+        """True if every operator acts along the lines through the solution
+        points, whose ends are the flux points."""
+        return self.on_lines and not self.surf_flux
+
+    @cached_property
+    def lines(self):
+        """The 1-D operators the full ones are made of: (d, hl, hr, ll, lr,
+        x) with d the line block of M1 - M3*M2, which is that of M4 - M6*M0
+        too; hl, hr the columns of M3 at the low and high end (M6: -hl, hr);
+        ll, lr the rows of M0."""
+        (ll, lr), (hl, hr) = ([v[s] for s in (-1, 1)]
+                              for v in (self.lend, self.hend))
+        d = self.dmat + np.outer(hl, ll) - np.outer(hr, lr)
+        return d, hl, hr, ll, lr, self.x1d
+
     # -- operators (layouts of pyfr/shapes.py:89-123)
     @cached_property
     def m0(self):

@@ -612,6 +612,47 @@ class EulerElements(FluidElements):
                     xa=self._xa_mats(xa), stage=stage)
             self.kernels['tdivf_flux'] = tdivf_flux
 
+        if self.hex_lines and type(self) is EulerElements:
+            gamma = self.cfg.getfloat('constants', 'gamma')
+
+            def hexdiv(uin, fout, xa=None, stage=None, disu=False):
+                return self._by_region(lambda mode, n, s, metric: be.kernel(
+                    'hexdiv', self.basis, mode, n, s(self.scal_upts[uin]),
+                    s(self._scal_fpts), s(self.scal_upts[fout]),
+                    s(self._rcpdjac_upts), gamma, metric,
+                    xa=self._xa_slices(xa, s), stage=stage, disu=disu,
+                    base=self.base_tpl.get('base')))
+            self.kernels['hexdiv'] = hexdiv
+
+    @property
+    def hex_lines(self):
+        """True if the element's passes run in the line kernels of hexes:
+        Gauss-Legendre solution points, no anti-aliasing, p <= 4, and the
+        flux folded into the divergence wherever it can be."""
+        be = self._be
+        return (self.name == 'hex' and self.basis.has_lines and
+                self.basis.n <= 5 and not self.fluxaa and be.fuse_flux and
+                not be.ops_bf16)
+
+    def _by_region(self, make):
+        """make(geometry mode, elements, slicer, metric terms) for each of
+        the curved and linear regions."""
+        ks = []
+        for region, n in self.mesh_regions.items():
+            lin = region == 'linear'
+            whole = len(self.mesh_regions) == 1
+
+            def s(m, region=region, whole=whole):
+                return m if whole else self._slice_mat(m, region)
+            ks.append(make(int(lin), n, s, self._verts_linear if lin
+                           else self._smats_curved))
+        return ks[0] if len(ks) == 1 else self._be.unordered_meta_kernel(ks)
+
+    def _xa_slices(self, xa, s):
+        xa = self._xa_mats(xa)
+        return (None if xa is None else
+                tuple(s(m) for m in xa) if isinstance(xa, tuple) else s(xa))
+
 
 class NavierStokesElements(EulerElements):
     @property
@@ -1383,10 +1424,10 @@ class BaseSystem:
             self._kcache[key] = g or self._build_graphs(uin, fout)
         return self._kcache[key]
 
-    def _try_fused(self, uin, fout, xa=None, stage=None):
+    def _try_fused(self, uin, fout, xa=None, stage=None, **kw):
         from pyfr_amd.backend import NotSuitableError, flat_kernels
         try:
-            ks = self._fused_kernels(uin, fout, xa, stage)
+            ks = self._fused_kernels(uin, fout, xa, stage, **kw)
         except NotSuitableError:
             return None
         g = self.backend.graph()
@@ -1411,15 +1452,20 @@ class BaseSystem:
                 self._fused_ok = False
         return self._fused_ok
 
-    def rhs_stage(self, t, uin, fout, xa, stage, dta, dtb, last, mixed=False):
+    def rhs_stage(self, t, uin, fout, xa, stage, dta, dtb, last, mixed=False,
+                  traced=False, trace=False):
         """RHS into fout fused with the rkvdh2 stage update
         (``rkvdh2.mako:4-31``): xa' = xa + dta*k, fout' = xa + dtb*k (if last,
         only xa' = xa + dtb*k).  mixed: xa is the FP64 accumulated solution
-        and fout the FP32 stage input."""
-        key = (uin, fout, xa, stage, mixed)
+        and fout the FP32 stage input.  trace: element types whose kernels
+        can leave the next stage's traces (disu of its input: xa', or fout'
+        in the precision form) in the flux-point buffer; traced: the stage
+        before did so for uin."""
+        key = (uin, fout, xa, stage, mixed, traced, trace)
         if key not in self._kcache:
             self._kcache[key] = self._try_fused(
-                uin, fout, xa, 'rk45-mixed' if mixed else 'rk45')
+                uin, fout, xa, 'rk45-mixed' if mixed else 'rk45',
+                traced=traced, trace=trace)
         self._set_time(t, uin)
         for g in self._kcache[key]:
             for k in g.stage_kernels:
@@ -1453,17 +1499,20 @@ class BaseSystem:
     def fused_rk4_mixed(self):
         return self._fused_rk4_ok(True)
 
-    def rhs_rk4_stage(self, t, stage, uin, nxt, r1, r0, dt, mixed=False):
+    def rhs_rk4_stage(self, t, stage, uin, nxt, r1, r0, dt, mixed=False,
+                      traced=False, trace=False):
         """RHS of RK4 stage `stage` at t with the stage's register updates
         in the divergence kernel's epilogue (``steppers.py:67-108``; mixed:
         the precision form's FP64 updates).  The epilogues read dt from
         device memory (bind writes it on the stream), so each stage's graph
-        is captured once, whatever the steps before an output time."""
+        is captured once, whatever the steps before an output time.
+        traced, trace: as for ``rhs_stage``."""
         from pyfr_amd.backend import flat_kernels
-        key = ('rk4', stage, uin, nxt, r1, r0, mixed)
+        key = ('rk4', stage, uin, nxt, r1, r0, mixed, traced, trace)
         if key not in self._kcache:
             ks = self._fused_kernels(uin, nxt, (r1, r0),
-                                     f'rk4{"m" if mixed else ""}-{stage}')
+                                     f'rk4{"m" if mixed else ""}-{stage}',
+                                     traced=traced, trace=trace)
             g = self.backend.graph()
             g.add_all(ks)
             g.commit()
@@ -1562,16 +1611,23 @@ class EulerSystem(BaseSystem):
     intinterscls = EulerIntInters
     bcinterscls = EulerBCInters
 
-    def _fused_kernels(self, uin, fout, xa, stage):
+    def _fused_kernels(self, uin, fout, xa, stage, traced=False, trace=False):
         """The fused RHS as kernels and Concurrent groups: the element
         types' kernels of one phase touch only their own arrays, so a
-        captured graph runs them side by side."""
+        captured graph runs them side by side.  traced: the line kernels'
+        element types have the traces of uin already; trace: they leave
+        those of the next stage's input."""
         from pyfr_amd.backend import Concurrent, NotSuitableError
         eles = list(self.ele_map.values())
-        ks = [Concurrent([[e.kernels['disu'](uin)] for e in eles])]
+        ks = [Concurrent([[e.kernels['disu'](uin)] for e in eles
+                          if not (traced and 'hexdiv' in e.kernels)])]
         ks += [i.kernels['comm_flux']() for i in self._inters]
         chains = []
         for e in eles:
+            if 'hexdiv' in e.kernels:
+                chains.append([e.kernels['hexdiv'](uin, fout, xa, stage,
+                                                   trace)])
+                continue
             if 'tdivf_flux' in e.kernels:
                 try:
                     chains.append([e.kernels['tdivf_flux'](uin, fout, xa,
@@ -1614,7 +1670,7 @@ class NavierStokesSystem(BaseSystem):
         return [e.kernels['copy_fpts']() for e in eles
                 if 'copy_fpts' in e.kernels]
 
-    def _fused_kernels(self, uin, fout, xa, stage):
+    def _fused_kernels(self, uin, fout, xa, stage, traced=False, trace=False):
         from pyfr_amd.backend import Concurrent
         eles = list(self.ele_map.values())
         ks = [Concurrent([[e.kernels['disu'](uin)] + self._copy_fpts([e])
@@ -1762,10 +1818,10 @@ class RK4Integrator(BaseIntegrator):
             # stage inputs alternate between r2 and r3, so no stage reads
             # and writes one bank
             st = self.system.rhs_rk4_stage
-            st(t, 1, r0, r2, r1, r0, dt)
-            st(t + dt/2.0, 2, r2, r3, r1, r0, dt)
-            st(t + dt/2.0, 3, r3, r2, r1, r0, dt)
-            st(t + dt, 4, r2, r2, r1, r0, dt)
+            st(t, 1, r0, r2, r1, r0, dt, trace=True)
+            st(t + dt/2.0, 2, r2, r3, r1, r0, dt, traced=True, trace=True)
+            st(t + dt/2.0, 3, r3, r2, r1, r0, dt, traced=True, trace=True)
+            st(t + dt, 4, r2, r2, r1, r0, dt, traced=True)
             self.nrhsevals += 4
             return r1
         rhs(t, r0, r1)
@@ -1813,10 +1869,12 @@ class MixedRK4Integrator(BaseIntegrator):
             self._sync_work(r0)
         if self.system.fused_rk4_mixed:
             st = self.system.rhs_rk4_stage
-            st(t, 1, wa, wb, r1, r0, dt, mixed=True)
-            st(t + dt/2.0, 2, wb, wa, r1, r0, dt, mixed=True)
-            st(t + dt/2.0, 3, wa, wb, r1, r0, dt, mixed=True)
-            st(t + dt, 4, wb, wa, r1, r0, dt, mixed=True)
+            st(t, 1, wa, wb, r1, r0, dt, mixed=True, trace=True)
+            st(t + dt/2.0, 2, wb, wa, r1, r0, dt, mixed=True, traced=True,
+               trace=True)
+            st(t + dt/2.0, 3, wa, wb, r1, r0, dt, mixed=True, traced=True,
+               trace=True)
+            st(t + dt, 4, wb, wa, r1, r0, dt, mixed=True, traced=True)
             self.nrhsevals += 4
             return r1
         lib, be = self.backend.lib, self.backend
@@ -1872,7 +1930,8 @@ class RK45Integrator(BaseIntegrator):
                 # RHS with the stage update in its final kernel
                 self.system.rhs_stage(t + ci*dt, uin, r2, r1, i,
                                       dt*self.a[i] if i < last else 0.0,
-                                      dt*self.b[i], i == last)
+                                      dt*self.b[i], i == last,
+                                      traced=i > 0, trace=i < last)
                 self.nrhsevals += 1
             else:
                 self._rhs(t + ci*dt, uin, r2)
@@ -1916,7 +1975,8 @@ class MixedRK45Integrator(RK45Integrator):
             dtb = dt*self.b[i]
             if fused:
                 self.system.rhs_stage(t + ci*dt, 1, 1, 0, i, dta, dtb,
-                                      i == last, mixed=True)
+                                      i == last, mixed=True, traced=i > 0,
+                                      trace=i < last)
                 self.nrhsevals += 1
                 continue
             self._rhs(t + ci*dt, 1, 1)

@@ -1,0 +1,119 @@
+"""Line kernels of hexahedra: their 1-D operators against the full ones, and
+the passes that run in them against the kernel sequences they replace."""
+import numpy as np
+import pytest
+
+from pyfr_amd.mesh import BoxMesh
+from pyfr_amd.shapes import HEX_FACES, HexShape
+from pyfr_amd.solvers import get_integrator
+from tests.fr_cases import make_cfg, rel_l2
+
+
+@pytest.mark.parametrize('order', [1, 2, 3, 4])
+def test_lines_make_the_operators(order):
+    """M0, M3, M6 and the corrected derivatives, rebuilt from the lines."""
+    sh = HexShape(order)
+    d, hl, hr, ll, lr, _ = sh.lines
+    n, nu = sh.n, sh.nupts
+    m0, m3 = np.zeros((sh.nfpts, nu)), np.zeros((nu, sh.nfpts))
+    m6 = np.zeros((3*nu, sh.nfpts))
+    for f, (nax, side, _, _) in enumerate(HEX_FACES):
+        for b in range(n):
+            for a in range(n):
+                line, row = sh.fpt_line(f, a, b)[0], f*n*n + a + n*b
+                m0[row, line] = lr if side > 0 else ll
+                m3[line, row] = hr if side > 0 else hl
+                m6[nax*nu + np.array(line), row] = side*m3[line, row]
+    div = np.zeros((nu, 3*nu))
+    for p in range(nu):
+        c = [p % n, p//n % n, p//(n*n)]
+        for ax in range(3):
+            for m in range(n):
+                q = list(c)
+                q[ax] = m
+                div[p, ax*nu + sh.uidx(*q)] = d[c[ax], m]
+    grad = div.reshape(nu, 3, nu).swapaxes(0, 1).reshape(3*nu, nu)
+    for got, expr in ((m0, 'M0'), (m3, 'M3'), (m6, 'M6'),
+                      (div, 'M1 - M3*M2'), (grad, 'M4 - M6*M0')):
+        ref = sh.opmat(expr)
+        # sums of a few products of entries up to about 30
+        assert np.abs(got - ref).max() < 1e-13, expr
+
+
+def _warp(x, y, z):
+    """Moves the low-x half only: curved elements there, linear beyond."""
+    s = np.where(x < 3.0, 0.05*np.sin(x)**2*np.sin(y)*np.sin(z), 0.0)
+    return x + s, y - s, z + 0.5*s
+
+
+def _run(make, system, n, order, fuse, scheme=None, steps=2, kind='straight',
+         precision='double'):
+    be = make(precision=precision, fuse_flux=fuse)
+    cfg = make_cfg(system, order, precision=precision,
+                   scheme=scheme or 'rk4', dt=1e-3)
+    kw = {}
+    if kind == 'skew':
+        kw = {'warp': lambda x, y, z: (x + 0.05*np.sin(y), y, z)}
+    elif kind == 'mixed':
+        kw = {'sorder': 2, 'warp': _warp}
+    integ = get_integrator(be, BoxMesh(n, **kw), cfg)
+    sysm = integ.system
+    if scheme is None:
+        sysm.rhs(0.0, 0, 1)
+        return sysm.ele_scal_upts(1)[0], sysm
+    integ.run_steps(steps, 1e-3)
+    return integ.soln[0], sysm
+
+
+def _rms(a):
+    return float(np.sqrt(np.mean(np.square(a))))
+
+
+def _rounding(n, order):
+    """Rounding error of a right-hand side: its terms are fluxes of up to
+    250 (of E, at p = 71.5) times 2/h = n/pi times 1-D derivatives whose
+    rows sum to 2(p + 1)^2 in modulus; eight roundings of each."""
+    return 8*2.2e-16*250*max(n)/np.pi*2*(order + 1)**2
+
+
+# 60 elements end in a partial block; the larger meshes reach the blocks of
+# more than 16 elements that grids of 256 blocks and over take
+SIZES = [((5, 4, 3), o) for o in (1, 2, 3, 4)] + \
+        [((26, 26, 25), 1), ((26, 26, 25), 2)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('n,order,kind', [
+    (n, o, k) for n, o in SIZES for k in ('straight', 'skew')] + [
+    ((6, 6, 6), 2, 'mixed'), ((6, 6, 6), 3, 'mixed')])
+def test_euler_rhs(backend_factory, n, order, kind):
+    """Flux, divergence and correction in one kernel, on straight, skewed
+    and part curved meshes."""
+    print(f'\n[hexline rhs] {n} p={order} {kind}', flush=True)
+    got, sysm = _run(backend_factory, 'euler', n, order, True, kind=kind)
+    ref, _ = _run(backend_factory, 'euler', n, order, False, kind=kind)
+    if kind == 'mixed':
+        assert len(sysm.ele_map['hex'].mesh_regions) == 2
+    assert _rms(got - ref) < _rounding(n, order)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('scheme', ['rk4', 'rk45', 'rk34', 'euler'])
+@pytest.mark.parametrize('precision', ['double', 'single', 'mixed'])
+@pytest.mark.parametrize('n,order', [((5, 4, 3), 1), ((5, 4, 3), 3),
+                                     ((21, 21, 19), 4), ((26, 26, 25), 3)])
+def test_euler_steps(backend_factory, scheme, precision, n, order):
+    """The stage updates, and the traces of the next stage's input left by
+    the kernel that forms it."""
+    if precision == 'mixed' and scheme == 'euler':
+        pytest.skip('no such stepper')
+    if n[0] > 5 and (precision == 'double' or scheme in ('rk34', 'euler')):
+        pytest.skip('these blocks are only taken in single precision')
+    print(f'\n[hexline step] {n} p={order} {scheme} {precision}', flush=True)
+    got, _ = _run(backend_factory, 'euler', n, order, True, scheme,
+                  precision=precision)
+    ref, _ = _run(backend_factory, 'euler', n, order, False, scheme,
+                  precision=precision)
+    # two steps: rounding of the state, and the right-hand side's in dt
+    tol = {'double': 1e-14, 'single': 2e-6, 'mixed': 1e-6}[precision]
+    assert rel_l2(got, ref) < tol
