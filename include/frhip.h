@@ -189,6 +189,23 @@ int frhip_hex_div(void *plan, int geo, int neles, const void *u, long ldu,
                   double dta, double dtb, int last, int disu, double gamma,
                   const double *base, void *stream);
 
+/* Navier-Stokes volume pass: tgradpcoru + tgradcoru (pyfr/solvers/
+ * baseadvecdiff/elements.py:47-55) + tdisf fused (pyfr/solvers/navstokes/
+ * kernels/tflux.mako:13-50) + tdivtpcorf + gradcoru_fpts (baseadvecdiff/
+ * elements.py:87-101).  u (n^3, 5, neles), cm (6 n^2, 5, neles) the common
+ * solution; gm, rcp the metric terms (rcp: geo = FRHIP_GEO_CURVED); dv
+ * (n^3, 5, neles) receives the volume part of the transformed divergence
+ * and g the physical gradients at the flux points (3, 6 n^2, 5, neles),
+ * which may hold cm in its first 6 n^2 rows, or, with nfv (linear hexes),
+ * (6 n^2, 5, neles): the viscous flux along the element's own unnormalised
+ * outward normal (variable 0, which has none, is not written).  consts and
+ * base: as frhip_tflux_ns. */
+int frhip_hex_nsvol(void *plan, int geo, int neles, const void *u, long ldu,
+                    const void *cm, long ldcm, const void *gm, long ldg,
+                    const void *rcp, long ldr, void *dv, long ldd, void *g,
+                    long ldgr, int nfv, const double *consts,
+                    const double *base, void *stream);
+
 /* ---- flux-fused divergence for straight-sided tets and prisms (Euler):
  *      tdisf (pyfr/solvers/euler/kernels/tflux.mako:8-30) + tdivtpcorf +
  *      tdivtconf + negdivconf (pyfr/solvers/baseadvec/elements.py:84-119)
@@ -328,6 +345,14 @@ int frhip_intcflux_ns(int dtype, int rsolver, int n, void *ubase,
                       const void *nl, long ldn, const double *consts,
                       double pmin, const void *mu_p, const double *bstate,
                       void *stream);
+/* The same from each side's normal viscous flux (frhip_hex_nsvol, nfv) at
+ * vbase + lmap[i], vbase + rmap[i]; the two sides' normals must be opposite
+ * to rounding. */
+int frhip_intcflux_nfv(int dtype, int rsolver, int n, void *ubase,
+                       const int32_t *lmap, const int32_t *rmap,
+                       const void *vbase, const void *nl, long ldn,
+                       const double *consts, double pmin,
+                       const double *bstate, void *stream);
 
 /* ---- boundary interfaces, 1-D over n boundary flux points ----
  * Types: the `type` keys of [soln-bcs-*] (pyfr/solvers/euler/inters.py:57-102,

@@ -915,6 +915,30 @@ class HexLineProvider:
         k.disu = disu
         return k
 
+    def hexns(self, basis, geo, neles, u, comm, dv, grad, tplargs, metric,
+              rcpdjac, nfv=False):
+        """tgradpcoru + tgradcoru + tdisf + tdivtpcorf + gradcoru_fpts over
+        neles elements: dv's first nupts rows receive the volume divergence,
+        grad the gradients at the flux points or (nfv) its second nfpts rows
+        each side's normal viscous flux."""
+        nu, nf = basis.nupts, basis.nfpts
+        if (u.nrow != nu or comm.nrow < nf or dv.nrow < nu or
+                grad.nrow != 3*nf or any(m.ncol != u.ncol or
+                                         m.dtype != u.dtype
+                                         for m in (comm, dv, grad))):
+            raise ValueError('Incompatible matrices for hexns')
+        plan = self._plan(basis, u.dtype)
+        base = PointwiseProvider._base(tplargs)
+        consts = PointwiseProvider._ns_consts(tplargs)
+        gp = grad.data + (nf*grad.leaddim*grad.itemsize if nfv else 0)
+        args = (plan, geo, neles, u.data, u.leaddim, comm.data, comm.leaddim,
+                metric.data, metric.leaddim, rcpdjac.data, rcpdjac.leaddim,
+                dv.data, dv.leaddim, gp, grad.leaddim, int(nfv), consts, base)
+        lib = self.backend.lib
+        return Kernel(lambda stream: lib.hex_nsvol(*args, stream),
+                      mats=(u, comm, dv, grad, metric),
+                      name=f'hexns{"_nfv" if nfv else ""}')
+
     def __del__(self):
         try:
             for plan in self._plans.values():
@@ -1118,6 +1142,15 @@ class PointwiseProvider:
         b = tplargs.get('base')
         return None if b is None else (ct.c_double*2)(*b)
 
+    @staticmethod
+    def _ns_consts(tplargs):
+        c = tplargs['c']
+        return (ct.c_double*8)(
+            c['gamma'], c.get('mu', 0.0), c.get('Pr', 1.0),
+            c.get('ldg-beta', 0.0), c.get('ldg-tau', 0.0),
+            1.0 if tplargs.get('visc_corr') == 'sutherland' else 0.0,
+            c.get('cpTref', 1.0), c.get('cpTs', 0.0))
+
     # -- tflux (Euler and NS) ------------------------------------------------
     def tflux(self, tplargs, dims, u, f, smats=None, verts=None, upts=None,
               gradu=None, rcpdjac=None, artvisc_vtx=None, **kw):
@@ -1134,11 +1167,7 @@ class PointwiseProvider:
         c = tplargs['c']
         ns = 'visc_corr' in tplargs
         if ns:
-            consts = (ct.c_double*8)(
-                c['gamma'], c.get('mu', 0.0), c.get('Pr', 1.0),
-                c.get('ldg-beta', 0.0), c.get('ldg-tau', 0.0),
-                1.0 if tplargs.get('visc_corr') == 'sutherland' else 0.0,
-                c.get('cpTref', 1.0), c.get('cpTs', 0.0))
+            consts = self._ns_consts(tplargs)
         if ns and 'fused' not in ktype:
             if base is not None:
                 raise NotSuitableError('the base-state form has no unfused '
@@ -1207,7 +1236,10 @@ class PointwiseProvider:
         return -1.0 if pm is None else float(pm)
 
     def intcflux(self, tplargs, dims, ul, ur, nl, gradul=None, gradur=None,
-                 artvisc=None, **kw):
+                 artvisc=None, nfv=False, **kw):
+        """Common flux of internal interfaces.  nfv: the second nfpts rows
+        of the views gradul, gradur hold each side's normal viscous flux
+        (``HexLineProvider.hexns``)."""
         lib = self.backend.lib
         (n,) = dims
         if ul.basedata != ur.basedata:
@@ -1228,10 +1260,21 @@ class PointwiseProvider:
         if artvisc is not None:
             raise NotSuitableError('artificial viscosity is not supported')
         gs = View.stride_args(gradul, gradur)
-        consts = (ct.c_double*8)(
-            c['gamma'], c['mu'], c['Pr'], c['ldg-beta'], c['ldg-tau'],
-            1.0 if tplargs.get('visc_corr') == 'sutherland' else 0.0,
-            c.get('cpTref', 1.0), c.get('cpTs', 0.0))
+        consts = self._ns_consts(tplargs)
+        if nfv:
+            # one map serves both arrays where they differ by an offset
+            delta = set(np.unique(gradul.mapping_np - ul.mapping_np)) | \
+                set(np.unique(gradur.mapping_np - ur.mapping_np))
+            if len(delta) != 1 or gs[1] is not None:
+                raise NotSuitableError('needs one element type')
+            vb = gradul.basedata + (int(delta.pop()) + gs[0])*np.dtype(
+                ul.refdtype).itemsize
+            args = (dt, rs, n, ul.basedata, ul.mapping.data, ur.mapping.data,
+                    vb, nl.data, nl.leaddim, consts, self._pmin(tplargs),
+                    base)
+            return Kernel(lambda stream: lib.intcflux_nfv(*args, stream),
+                          views=(ul, ur, gradul, gradur), mats=(nl,),
+                          name='intcflux_nfv')
         args = (dt, rs, n, ul.basedata, ul.mapping.data, ur.mapping.data,
                 gradul.basedata, gradul.mapping.data, gradur.mapping.data,
                 *gs, nl.data, nl.leaddim, consts, self._pmin(tplargs), None,

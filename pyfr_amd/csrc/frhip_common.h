@@ -61,6 +61,17 @@ __host__ __device__ inline long soa_ix(long e, int v, int nvar)
     return ((e >> 6) * nvar + v) * SOA + (e & 63);
 }
 
+// Workgroup index with each XCD given a contiguous range: workgroups are
+// dispatched to the 8 XCDs round-robin (block b to XCD b % 8), so
+// consecutive indices, whose wavefronts read the same element block's data,
+// would otherwise sit in different L2s and fetch it from HBM once each.
+__device__ __forceinline__ unsigned xcd_block()
+{
+    const unsigned b = blockIdx.x, nb = gridDim.x;
+    const unsigned per = nb/8, rem = nb % 8, x = b % 8;
+    return x*per + min(x, rem) + b/8;
+}
+
 inline hipStream_t as_stream(void *s) { return static_cast<hipStream_t>(s); }
 
 inline unsigned int cdiv(long a, long b) { return (unsigned int)((a + b - 1) / b); }

@@ -25,8 +25,10 @@
 // gradcoru_fpts; writes the volume divergence and, at the flux points, the
 // gradients or only the normal viscous flux each side contributes.
 //
-// All are bound by HBM: an FP64 p = 3 element moves 416 x 40 B in
-// k_hex_nsvol at about 3.5 flop/B.
+// k_hex_div is bound by HBM (4.2-4.8 TB/s).  k_hex_nsvol moves 301 x 40 B of
+// an FP64 p = 3 element (1.33 GB on 48^3, by counters as by count; the four
+// kernels replaced moved 1600 x 40 B) and is bound by issue: 1,107 vector
+// and 180 LDS instructions a wavefront, 44 % and 34 % of its cycles.
 #include "frhip_common.h"
 #include "frhip_physics.h"
 
@@ -513,6 +515,336 @@ __attribute__((amdgpu_waves_per_eu(
 }
 
 // ---------------------------------------------------------------------------
+// Navier-Stokes volume pass
+// ---------------------------------------------------------------------------
+
+template <typename T>
+struct HexNsArgs {
+    int neles;
+    const T *u;
+    long ldu;
+    const T *cm;        // common solution at the flux points
+    long ldcm;
+    const T *geo;
+    long ldg;
+    const T *rcp;
+    long ldr;
+    T *dv;              // volume part of the transformed divergence
+    long ldd;
+    T *g;               // gradients (3, nfpts, 5, E) or normal viscous flux
+    long ldgr;
+    NSConsts<T> c;
+    BaseState<T> bs;
+};
+
+// Five variables at NP points of EB elements in LDS, as many of them side by
+// side as 16 B hold, so that most accesses are ds_read_b128: an 8 B read
+// takes as many LDS cycles as a 16 B one (k_hex_nsvol, FP64 p = 3, 48^3:
+// 596 us with a plane per variable).
+template <typename T, int NP, int EB>
+struct Lds5 {
+    static constexpr int W = 16/sizeof(T), G = 5/W, R = 5 - G*W;
+    typedef T V __attribute__((ext_vector_type(W)));
+
+    static __device__ __forceinline__ void load(const T *b, int p, int el,
+                                                T (&x)[5])
+    {
+        const int q = p*EB + el;
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            const V v = *reinterpret_cast<const V *>(b + (g*NP*EB + q)*W);
+#pragma unroll
+            for (int w = 0; w < W; ++w) x[g*W + w] = v[w];
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) x[G*W + r] = b[(G*W + r)*NP*EB + q];
+    }
+
+    static __device__ __forceinline__ void store(T *b, int p, int el,
+                                                 const T (&x)[5])
+    {
+        const int q = p*EB + el;
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            V v;
+#pragma unroll
+            for (int w = 0; w < W; ++w) v[w] = x[g*W + w];
+            *reinterpret_cast<V *>(b + (g*NP*EB + q)*W) = v;
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) b[(G*W + r)*NP*EB + q] = x[G*W + r];
+    }
+};
+
+// y += l x
+template <typename T>
+__device__ __forceinline__ void fma5(T l, const T (&x)[5], T (&y)[5])
+{
+#pragma unroll
+    for (int v = 0; v < 5; ++v) y[v] = fma(l, x[v], y[v]);
+}
+
+// The two in-plane axes of face axis a and the faces of its sides
+// (HEX_FACES, pyfr/shapes.py:378-385)
+struct HexFace {
+    int axis, side, a, b;       // flux point (a, b), first coordinate first
+
+    template <int N>
+    static __device__ __forceinline__ HexFace of(int q)
+    {
+        const int f = q/(N*N), r = q - f*N*N;
+        HexFace h;
+        h.axis = f == 0 || f == 5 ? 2 : f == 1 || f == 3 ? 1 : 0;
+        h.side = f == 2 || f == 3 || f == 5;
+        h.b = r/N;
+        h.a = r - h.b*N;
+        return h;
+    }
+
+    // first solution point of the line that ends here, and its step
+    template <int N>
+    __device__ __forceinline__ void line(int &p0, int &step) const
+    {
+        p0 = axis == 0 ? N*(a + N*b) : axis == 1 ? a + N*N*b : a + N*b;
+        step = axis == 0 ? 1 : axis == 1 ? N : N*N;
+    }
+};
+
+// One thread per (solution point, element).  The element's u and common
+// solution, then the transformed flux, then the gradients pass through one
+// LDS buffer; all of the (3, Nu, 5) and (3, Nf, 5) intermediates of the
+// kernels replaced stay in registers and LDS.  NFV: at the flux points only
+// the normal viscous flux of this side (4 values) instead of the gradients
+// (15), for meshes whose interface kernel needs no more.
+template <typename T, int N, int GEO, bool NFV, int EB>
+__global__ __launch_bounds__(N*N*N*EB)
+__attribute__((amdgpu_waves_per_eu(4))) void k_hex_nsvol(
+    const HexLine<T, N> *__restrict__ line, HexNsArgs<T> a)
+{
+    constexpr int NN = N*N, NU = N*NN, NF = 6*NN;
+    constexpr int SLOTS = (NF + NU - 1)/NU;
+    // u, and one buffer for the common solution (5 NF), then the flux, then
+    // the gradients (15 NU each)
+    static_assert(5*NF <= 15*NU, "LDS layout");
+    __shared__ __attribute__((aligned(16))) T sh[20*NU*EB];
+
+    const int el = threadIdx.x % EB, pt = threadIdx.x/EB;
+    const int i = pt % N, j = pt/N % N;
+    // uniform where a layer of constant z is whole wavefronts
+    const int k = NN*EB % 64 ? pt/NN
+                             : __builtin_amdgcn_readfirstlane(pt/NN);
+    const int e = xcd_block()*EB + el;
+    const bool ok = e < a.neles;
+    const long col = soa_ix(e, 0, 5);
+
+    T u[5];
+    const T *pu = a.u + pt*a.ldu + col;
+#pragma unroll
+    for (int v = 0; v < 5; ++v) u[v] = pu[v*SOA];
+    T cm[SLOTS][5];
+#pragma unroll
+    for (int s = 0; s < SLOTS; ++s) {
+        const int q = pt + s*NU;
+        if (q < NF)
+#pragma unroll
+            for (int v = 0; v < 5; ++v)
+                cm[s][v] = a.cm[q*a.ldcm + col + v*SOA];
+    }
+
+    using Lu = Lds5<T, NU, EB>;
+    using Lf = Lds5<T, NF, EB>;
+    T *su = sh, *sb = sh + 5*NU*EB;
+    Lu::store(su, pt, el, u);
+#pragma unroll
+    for (int s = 0; s < SLOTS; ++s) {
+        const int q = pt + s*NU;
+        if (q < NF) Lf::store(sb, q, el, cm[s]);
+    }
+    layer_end(u);
+
+    // metric terms at this point
+    T S[3][3], rj[1];
+    if constexpr (GEO == FRHIP_GEO_HEX_LINEAR) {
+        PencilGeo<T> pg;
+        T d;
+        pg.load(a.geo, a.ldg, (unsigned)soa_ix(e, 0, 3)*(unsigned)sizeof(T),
+                line->x[i], line->x[j]);
+        pg.smats(line->x[k], S, d);
+        rj[0] = T(1)/d;
+    }
+    else {
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+#pragma unroll
+            for (int c = 0; c < 3; ++c)
+                S[q][c] = a.geo[((long)q*NU + pt)*a.ldg + soa_ix(e, c, 3)];
+        rj[0] = a.rcp[pt*a.ldr + e];
+    }
+
+    lds_barrier();
+
+    // corrected gradient, made physical (transform_grad.mako:3-10)
+    T g[3][5];
+    {
+        T cx[N], cy[N], cz[N];
+#pragma unroll
+        for (int m = 0; m < N; ++m) {
+            cx[m] = line->d[i][m];
+            cy[m] = line->d[j][m];
+            cz[m] = line->d[k][m];
+        }
+        const T hx[2] = {-line->hl[i], line->hr[i]};
+        const T hy[2] = {-line->hl[j], line->hr[j]};
+        const T hz[2] = {-line->hl[k], line->hr[k]};
+        const int px = N*(j + N*k), py = i + NN*k, pz = i + N*j;
+        const int qx = j + N*k, qy = i + N*k, qz = i + N*j;
+        using Rows = HexRows<N>;
+        T r[3][5] = {}, w[5];
+#pragma unroll
+        for (int m = 0; m < N; ++m) {
+            Lu::load(su, px + m, el, w);
+            fma5(cx[m], w, r[0]);
+            Lu::load(su, py + N*m, el, w);
+            fma5(cy[m], w, r[1]);
+            Lu::load(su, pz + NN*m, el, w);
+            fma5(cz[m], w, r[2]);
+        }
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            Lf::load(sb, Rows::x(s) + qx, el, w);
+            fma5(hx[s], w, r[0]);
+            Lf::load(sb, Rows::y(s) + qy, el, w);
+            fma5(hy[s], w, r[1]);
+            Lf::load(sb, Rows::z(s) + qz, el, w);
+            fma5(hz[s], w, r[2]);
+        }
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+#pragma unroll
+            for (int v = 0; v < 5; ++v)
+                g[d][v] = rj[0]*(S[0][d]*r[0][v] + S[1][d]*r[1][v] +
+                                 S[2][d]*r[2][v]);
+            layer_end(g[d]);
+        }
+    }
+
+    lds_barrier();              // the common solution has been read
+#pragma unroll
+    for (int d = 0; d < 3; ++d) Lu::store(sb + 5*d*NU*EB, pt, el, g[d]);
+    lds_barrier();
+#pragma unroll
+    for (int s = 0; s < SLOTS; ++s) {
+        const int q = pt + s*NU;
+        if (q >= NF) continue;
+        const HexFace h = HexFace::of<N>(q);
+        int p0, st;
+        h.line<N>(p0, st);
+        // this side's normal from the tangents along the face's axes (its
+        // four vertices), and its state
+        T nf[3] = {}, uf[5] = {};
+        if constexpr (NFV) {
+            T ts[3], tt[3];
+            const int sa = h.axis == 0 ? 1 : 0, ta = h.axis == 2 ? 1 : 2;
+            const int v0 = h.side << h.axis;
+            const T x = line->x[h.a], y = line->x[h.b];
+            const T *gv = a.geo + soa_ix(e, 0, 3);
+#pragma unroll
+            for (int b = 0; b < 3; ++b) {
+                const T w00 = gv[v0*a.ldg + b*SOA];
+                const T w10 = gv[(v0 | 1 << sa)*a.ldg + b*SOA];
+                const T w01 = gv[(v0 | 1 << ta)*a.ldg + b*SOA];
+                const T w11 = gv[(v0 | 1 << sa | 1 << ta)*a.ldg + b*SOA];
+                ts[b] = T(0.25)*((T(1) - y)*(w10 - w00) +
+                                 (T(1) + y)*(w11 - w01));
+                tt[b] = T(0.25)*((T(1) - x)*(w01 - w00) +
+                                 (T(1) + x)*(w11 - w10));
+            }
+            PencilGeo<T>::cross(ts, tt, nf);
+            // axes (y, z), (x, z), (x, y): the middle pair is left-handed
+            const T sg = (h.axis == 1) != (h.side == 0) ? T(-1) : T(1);
+#pragma unroll
+            for (int b = 0; b < 3; ++b) nf[b] *= sg;
+            layer_end(nf);
+#pragma unroll
+            for (int m = 0; m < N; ++m) {
+                T w[5];
+                Lu::load(su, p0 + st*m, el, w);
+                fma5(h.side ? line->lr[m] : line->ll[m], w, uf);
+            }
+            layer_end(uf);
+        }
+        T gf[3][5] = {};
+#pragma unroll
+        for (int m = 0; m < N; ++m) {
+            const T l = h.side ? line->lr[m] : line->ll[m];
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                T w[5];
+                Lu::load(sb + 5*d*NU*EB, p0 + st*m, el, w);
+                fma5(l, w, gf[d]);
+            }
+        }
+        T *pg = a.g + q*a.ldgr + col;
+        if constexpr (NFV) {
+#pragma unroll
+            for (int d = 0; d < 3; ++d) layer_end(gf[d]);
+            T w[5], f[3][5] = {};
+            base_full(uf, w, a.bs);
+            viscous_flux_add(w, gf, f, a.c);
+            if (ok)
+#pragma unroll
+                for (int v = 1; v < 5; ++v)
+                    pg[v*SOA] = nf[0]*f[0][v] + nf[1]*f[1][v] +
+                                nf[2]*f[2][v];
+        }
+        else if (ok)
+#pragma unroll
+            for (int d = 0; d < 3; ++d)
+#pragma unroll
+                for (int v = 0; v < 5; ++v)
+                    pg[(long)d*NF*a.ldgr + v*SOA] = gf[d][v];
+        layer_end(rj);
+    }
+
+    // the transformed flux
+    {
+        T w[5], f[3][5], p, vel[3];
+        Lu::load(su, pt, el, u);
+#pragma unroll
+        for (int d = 0; d < 3; ++d) Lu::load(sb + 5*d*NU*EB, pt, el, g[d]);
+        base_full(u, w, a.bs);
+        inviscid_flux_base(u, f, p, vel, a.c.gm1, a.bs);
+        viscous_flux_add(w, g, f, a.c);
+        lds_barrier();                      // the gradients have been read
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            T t[5];
+#pragma unroll
+            for (int v = 0; v < 5; ++v)
+                t[v] = S[d][0]*f[0][v] + S[d][1]*f[1][v] + S[d][2]*f[2][v];
+            Lu::store(sb + 5*d*NU*EB, pt, el, t);
+        }
+    }
+    lds_barrier();
+    {
+        T r[5] = {}, w[5];
+#pragma unroll
+        for (int m = 0; m < N; ++m) {
+            Lu::load(sb, N*(j + N*k) + m, el, w);
+            fma5(line->d[i][m], w, r);
+            Lu::load(sb + 5*NU*EB, i + NN*k + N*m, el, w);
+            fma5(line->d[j][m], w, r);
+            Lu::load(sb + 10*NU*EB, i + N*j + NN*m, el, w);
+            fma5(line->d[k][m], w, r);
+        }
+        T *pd = a.dv + pt*a.ldd + col;
+        if (ok)
+#pragma unroll
+            for (int v = 0; v < 5; ++v) pd[v*SOA] = r[v];
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Dispatch
 // ---------------------------------------------------------------------------
 
@@ -589,6 +921,53 @@ static int hex_div_t(const HexPlan *p, int geo, int neles, const void *u,
         case 3: return hex_div_n<T, 3>(p, geo, a, s);
         case 4: return hex_div_n<T, 4>(p, geo, a, s);
         default: return hex_div_n<T, 5>(p, geo, a, s);
+    }
+}
+
+// Elements per block of k_hex_nsvol: about 512 threads, so that two blocks
+// share a CU and one computes while the other loads (a wavefront holds 128
+// registers, a block 80 KB of LDS at p = 3 in FP64).  RK45 steps, 48^3 p = 3
+// FP64 with 8 / 4 elements 7.01 / 7.52 ms; 30^3 p = 4 FP64 3.66 / 3.38.
+template <typename T, int N>
+constexpr int hex_ns_eb()
+{
+    return N == 2 ? 64 : N == 3 ? 16 : N == 4 ? (sizeof(T) == 8 ? 8 : 16)
+                                              : (sizeof(T) == 8 ? 4 : 8);
+}
+
+template <typename T, int N>
+static int hex_ns_n(const HexPlan *p, int geo, int nfv, const HexNsArgs<T> &a,
+                    hipStream_t s)
+{
+    constexpr int EB = hex_ns_eb<T, N>();
+    const dim3 grid(cdiv(a.neles, EB)), block(N*N*N*EB);
+    const auto *line = static_cast<const HexLine<T, N> *>(p->line);
+    auto k = nfv ? k_hex_nsvol<T, N, FRHIP_GEO_HEX_LINEAR, true, EB>
+           : geo == FRHIP_GEO_HEX_LINEAR
+               ? k_hex_nsvol<T, N, FRHIP_GEO_HEX_LINEAR, false, EB>
+               : k_hex_nsvol<T, N, FRHIP_GEO_CURVED, false, EB>;
+    hipLaunchKernelGGL(k, grid, block, 0, s, line, a);
+    FR_LAUNCHED();
+    return 0;
+}
+
+template <typename T>
+static int hex_ns_t(const HexPlan *p, int geo, int nfv, int neles,
+                    const void *u, long ldu, const void *cm, long ldcm,
+                    const void *gm, long ldg, const void *rcp, long ldr,
+                    void *dv, long ldd, void *g, long ldgr,
+                    const double *consts, const double *base, hipStream_t s)
+{
+    const HexNsArgs<T> a{neles, (const T *)u, ldu, (const T *)cm, ldcm,
+                         (const T *)gm, ldg, (const T *)rcp, ldr, (T *)dv,
+                         ldd, (T *)g, ldgr, ns_consts<T>(consts, -1.0),
+                         base ? base_state<T>(base, consts[0])
+                              : BaseState<T>{}};
+    switch (p->n) {
+        case 2: return hex_ns_n<T, 2>(p, geo, nfv, a, s);
+        case 3: return hex_ns_n<T, 3>(p, geo, nfv, a, s);
+        case 4: return hex_ns_n<T, 4>(p, geo, nfv, a, s);
+        default: return hex_ns_n<T, 5>(p, geo, nfv, a, s);
     }
 }
 
@@ -674,6 +1053,34 @@ int frhip_hex_div(void *plan, int geo, int neles, const void *u, long ldu,
                             epi, rcp, ldr, xa, dta, dtb, disu, gamma, base, s)
         : hex_div_t<float>(p, geo, neles, u, ldu, gm, ldg, f, ldf, c, ldc,
                            epi, rcp, ldr, xa, dta, dtb, disu, gamma, base, s);
+    FR_API_END
+}
+
+int frhip_hex_nsvol(void *plan, int geo, int neles, const void *u, long ldu,
+                    const void *cm, long ldcm, const void *gm, long ldg,
+                    const void *rcp, long ldr, void *dv, long ldd, void *g,
+                    long ldgr, int nfv, const double *consts,
+                    const double *base, void *stream)
+{
+    FR_API_BEGIN
+    HexPlan *p = static_cast<HexPlan *>(plan);
+    FR_CHECK(p && u && cm && gm && dv && g && consts, "null argument");
+    FR_CHECK(geo == FRHIP_GEO_HEX_LINEAR ||
+             (geo == FRHIP_GEO_CURVED && rcp && !nfv),
+             "invalid geometry mode");
+    FR_CHECK(neles >= 0, "invalid extents");
+    const long ncol = 320L*((neles + 63L)/64);
+    FR_CHECK(ldu >= ncol && ldcm >= ncol && ldd >= ncol && ldgr >= ncol &&
+             ldg*5 >= ncol*3, "invalid leading dimensions");
+    // the vertices of a lane are addressed by 32-bit byte offsets
+    FR_CHECK((size_t)(neles + 63)*24 < (size_t)1 << 32, "too many elements");
+    if (neles == 0) return 0;
+    hipStream_t s = as_stream(stream);
+    return p->dtype == FRHIP_F64
+        ? hex_ns_t<double>(p, geo, nfv, neles, u, ldu, cm, ldcm, gm, ldg, rcp,
+                           ldr, dv, ldd, g, ldgr, consts, base, s)
+        : hex_ns_t<float>(p, geo, nfv, neles, u, ldu, cm, ldcm, gm, ldg, rcp,
+                          ldr, dv, ldd, g, ldgr, consts, base, s);
     FR_API_END
 }
 

@@ -393,6 +393,47 @@ __global__ __launch_bounds__(256) void k_intcflux_ns(
     }
 }
 
+// intcflux (NS) where each side's normal viscous flux is known
+// (k_hex_nsvol): vb holds it along the side's own unnormalised outward
+// normal, in the layout of base, so that with matching normals
+// mag*fvcomm = (1/2 + beta) vl - (1/2 - beta) vr.  Per pair 256 B in FP64
+// where the kernel above moves 440.
+template <typename T, int RS, bool BASE>
+__global__ __launch_bounds__(256) void k_intcflux_nfv(
+    int n, T *__restrict__ base, const int32_t *__restrict__ lmap,
+    const int32_t *__restrict__ rmap, const T *__restrict__ vb,
+    const T *__restrict__ nl, long ldn, NSConsts<T> c, BaseState<T> bs)
+{
+    const int i = blockIdx.x*blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const long li = lmap[i], ri = rmap[i];
+    T ul[5], ur[5], vl[5], vr[5];
+    for (int v = 0; v < 5; ++v) {
+        ul[v] = base[li + v*SOA];
+        ur[v] = base[ri + v*SOA];
+        vl[v] = v ? vb[li + v*SOA] : T(0);
+        vr[v] = v ? vb[ri + v*SOA] : T(0);
+    }
+    const T n0 = nl[i], n1 = nl[ldn + i], n2 = nl[2*ldn + i];
+    const T mag = sqrt((n0)*(n0) + (n1)*(n1) + (n2)*(n2));
+    const T nn[3] = {(T(1)/mag)*n0, (T(1)/mag)*n1, (T(1)/mag)*n2};
+    T fi[5];
+    if constexpr (BASE)
+        rsolve_rusanov_base(ul, ur, nn, fi, c.gm1, c.qgamma, bs);
+    else
+        rsolve<T, RS>(ul, ur, nn, fi, c.gm1, c.gamma, c.qgamma, c.pmin);
+    for (int v = 0; v < 5; ++v) {
+        T fv;
+        if (c.beta == T(-0.5)) fv = -vr[v];
+        else if (c.beta == T(0.5)) fv = vl[v];
+        else fv = (T(0.5) + c.beta)*vl[v] - (T(0.5) - c.beta)*vr[v];
+        if (c.tau != T(0)) fv += mag*(c.tau*(ul[v] - ur[v]));
+        const T f = mag*fi[v] + fv;
+        base[li + v*SOA] = f;
+        base[ri + v*SOA] = -f;
+    }
+}
+
 // ---------------------------------------------------------------------------
 // BLAS extensions
 // ---------------------------------------------------------------------------
@@ -845,6 +886,47 @@ int frhip_intcflux_ns(int dtype, int rsolver, int n, void *ubase,
 #undef FR_L64
 #undef FR_L32
 #undef FR_LNS
+    FR_LAUNCHED();
+    return 0;
+    FR_API_END
+}
+
+int frhip_intcflux_nfv(int dtype, int rsolver, int n, void *ubase,
+                       const int32_t *lmap, const int32_t *rmap,
+                       const void *vbase, const void *nl, long ldn,
+                       const double *consts, double pmin,
+                       const double *bstate, void *stream)
+{
+    FR_API_BEGIN
+    FR_DTYPE_OK(dtype);
+    FR_RS_OK(rsolver);
+    FR_CHECK(consts && vbase, "null argument");
+    FR_CHECK(!bstate || rsolver == FRHIP_RS_RUSANOV,
+             "the base-state form takes the Rusanov solver");
+    if (n == 0) return 0;
+    dim3 grid(cdiv(n, 256)), block(256);
+#define FR_LNV(T, RS, B, BS)                                                \
+    hipLaunchKernelGGL((k_intcflux_nfv<T, RS, B>), grid, block, 0,          \
+                       as_stream(stream), n, (T *)ubase, lmap, rmap,        \
+                       (const T *)vbase, (const T *)nl, ldn,                \
+                       ns_consts<T>(consts, pmin), BS)
+#define FR_L64(RS) FR_LNV(double, RS, false, BaseState<double>{})
+#define FR_L32(RS) FR_LNV(float, RS, false, BaseState<float>{})
+    if (bstate && dtype == FRHIP_F64)
+        FR_LNV(double, FRHIP_RS_RUSANOV, true,
+               base_state<double>(bstate, consts[0]));
+    else if (bstate)
+        FR_LNV(float, FRHIP_RS_RUSANOV, true,
+               base_state<float>(bstate, consts[0]));
+    else if (dtype == FRHIP_F64) {
+        FR_RS_DISPATCH(rsolver, FR_L64)
+    }
+    else {
+        FR_RS_DISPATCH(rsolver, FR_L32)
+    }
+#undef FR_L64
+#undef FR_L32
+#undef FR_LNV
     FR_LAUNCHED();
     return 0;
     FR_API_END

@@ -755,6 +755,24 @@ class NavierStokesElements(EulerElements):
             self.scal_upts[uin], self._comm_fpts, self._grad_upts)
         self._add_fused_kernels()
 
+        # hexes with line operators: everything between the common solution
+        # and the common flux in one pass, then the correction
+        if self.hex_lines:
+            def hexns(uin, nfv=False):
+                return self._by_region(lambda mode, n, s, metric: be.kernel(
+                    'hexns', self.basis, mode, n, s(self.scal_upts[uin]),
+                    s(self._vect_fpts), s(self._vect_upts),
+                    s(self._vect_fpts), tplargs | self.base_tpl, metric,
+                    s(self._rcpdjac_upts), nfv=nfv))
+
+            def hexdiv(fout, xa=None, stage=None, disu=False):
+                return be.kernel(
+                    'hexdiv', self.basis, -1, self.neles, self._vect_upts,
+                    self._scal_fpts, self.scal_upts[fout],
+                    self._rcpdjac_upts, xa=self._xa_mats(xa), stage=stage,
+                    disu=disu)
+            kernels['hexns'], kernels['hexdiv'] = hexns, hexdiv
+
     def _ns_flux_qpts(self, uin, tplargs):
         """Without gradient fusion (flux anti-aliasing): the corrected
         gradient made physical in place at the solution points (gradcoru,
@@ -921,10 +939,22 @@ class NavierStokesIntInters(EulerIntInters):
             'intconu', tplargs=self._tplargs, dims=[self.ninterfpts],
             ulin=self.scal_lhs, urin=self.scal_rhs, ulout=self._comm_lhs,
             urout=self._comm_rhs)
-        self.kernels['comm_flux'] = lambda: be.kernel(
+        self.kernels['comm_flux'] = lambda nfv=False: be.kernel(
             'intcflux', tplargs=self._tplargs, dims=[self.ninterfpts],
             ul=self.scal_lhs, ur=self.scal_rhs, gradul=self._vect_lhs,
-            gradur=self._vect_rhs, nl=self._pnorm_lhs)
+            gradur=self._vect_rhs, nl=self._pnorm_lhs, nfv=nfv)
+
+    @cached_property
+    def normals_match(self):
+        """True if the two sides' normals are opposite at every point to the
+        rounding of the stored metric (faces of the same vertices: 1e-12 of
+        a normal on 48^3 elements)."""
+        nl, nr = (_get_inter_arrays(i, 'get_pnorms_for_inters', self.elemap,
+                                    self._perm) for i in (self.lhs, self.rhs))
+        if not nl:
+            return True
+        mag = np.sqrt((nl[0]**2).sum(axis=1))
+        return bool(np.all(np.abs(nl[0] + nr[0]).max(axis=1) <= 1e-10*mag))
 
     def _gen_perm(self, scal):
         side = self.lhs if self._beta != -0.5 else self.rhs
@@ -1670,19 +1700,40 @@ class NavierStokesSystem(BaseSystem):
         return [e.kernels['copy_fpts']() for e in eles
                 if 'copy_fpts' in e.kernels]
 
+    @cached_property
+    def _nfv(self):
+        """True if the interfaces need no more than each side's normal
+        viscous flux: linear hexes only, whose shared faces have matching
+        normals, and no boundaries (their ghost states need gradients)."""
+        eles = list(self.ele_map.values())
+        return (len(eles) == 1 and eles[0].hex_lines and
+                not self._bc_inters and
+                set(eles[0].mesh_regions) == {'linear'} and
+                all(i.normals_match for i in self._int_inters))
+
     def _fused_kernels(self, uin, fout, xa, stage, traced=False, trace=False):
+        """traced, trace: as for EulerSystem."""
         from pyfr_amd.backend import Concurrent
         eles = list(self.ele_map.values())
-        ks = [Concurrent([[e.kernels['disu'](uin)] + self._copy_fpts([e])
-                          for e in eles])]
-        ks += [i.kernels['con_u']() for i in self._inters]
-        ks.append(Concurrent([[e.kernels['tgradf'](uin),
-                               e.kernels['tdisf_fused'](uin),
-                               e.kernels['gradcoru_fpts']()] for e in eles]))
-        ks += [i.kernels['comm_flux']() for i in self._inters]
-        ks.append(Concurrent([[e.kernels['tdivf'](fout, xa, stage)]
-                              for e in eles]))
-        return ks
+        pre, vol, post = [], [], []
+        for e in eles:
+            lines = 'hexdiv' in e.kernels
+            pre.append([] if traced and lines else [e.kernels['disu'](uin)])
+            pre[-1] += self._copy_fpts([e])
+            if lines:
+                vol.append([e.kernels['hexns'](uin, self._nfv)])
+                post.append([e.kernels['hexdiv'](fout, xa, stage, trace)])
+            else:
+                vol.append([e.kernels['tgradf'](uin),
+                            e.kernels['tdisf_fused'](uin),
+                            e.kernels['gradcoru_fpts']()])
+                post.append([e.kernels['tdivf'](fout, xa, stage)])
+        kw = {'nfv': True} if self._nfv else {}
+        return ([Concurrent(pre)] +
+                [i.kernels['con_u']() for i in self._inters] +
+                [Concurrent(vol)] +
+                [i.kernels['comm_flux'](**kw) for i in self._inters] +
+                [Concurrent(post)])
 
     def _build_graphs(self, uin, fout):
         """``pyfr/solvers/baseadvecdiff/system.py:53-231`` with gradient

@@ -47,10 +47,10 @@ def _warp(x, y, z):
 
 
 def _run(make, system, n, order, fuse, scheme=None, steps=2, kind='straight',
-         precision='double'):
+         precision='double', **cfgkw):
     be = make(precision=precision, fuse_flux=fuse)
     cfg = make_cfg(system, order, precision=precision,
-                   scheme=scheme or 'rk4', dt=1e-3)
+                   scheme=scheme or 'rk4', dt=1e-3, **cfgkw)
     kw = {}
     if kind == 'skew':
         kw = {'warp': lambda x, y, z: (x + 0.05*np.sin(y), y, z)}
@@ -117,3 +117,70 @@ def test_euler_steps(backend_factory, scheme, precision, n, order):
     # two steps: rounding of the state, and the right-hand side's in dt
     tol = {'double': 1e-14, 'single': 2e-6, 'mixed': 1e-6}[precision]
     assert rel_l2(got, ref) < tol
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('n,order,kind', [
+    ((5, 4, 3), o, k) for o in (1, 2, 3, 4) for k in ('straight', 'skew')] + [
+    ((6, 6, 6), 2, 'mixed'), ((6, 6, 6), 3, 'mixed')])
+@pytest.mark.parametrize('beta,tau,visc', [(0.0, 0.0, 'none'),
+                                           (0.5, 0.1, 'none'),
+                                           (-0.5, 0.0, 'none'),
+                                           (0.25, 0.1, 'none')])
+def test_ns_rhs(backend_factory, n, order, kind, beta, tau, visc):
+    """Gradient, flux and divergence in one kernel; linear meshes pass the
+    interfaces each side's normal viscous flux, part curved ones (and p = 1,
+    whose metric is stored) the gradients."""
+    print(f'\n[hexline ns] {n} p={order} {kind} {beta} {tau}', flush=True)
+    kw = dict(kind=kind, beta=beta, tau=tau, visc_corr=visc)
+    got, sysm = _run(backend_factory, 'navier-stokes', n, order, True, **kw)
+    assert sysm._nfv == (kind != 'mixed' and order > 1)
+    ref, _ = _run(backend_factory, 'navier-stokes', n, order, False, **kw)
+    # the viscous terms, a second derivative of fluxes of mu times order 1,
+    # stay below the inviscid ones
+    assert _rms(got - ref) < _rounding(n, order)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('scheme', ['rk4', 'rk45'])
+@pytest.mark.parametrize('precision', ['double', 'single', 'mixed'])
+@pytest.mark.parametrize('n,order', [((5, 4, 3), 2), ((5, 4, 3), 4),
+                                     ((9, 8, 8), 3)])
+def test_ns_steps(backend_factory, scheme, precision, n, order):
+    print(f'\n[hexline ns step] {n} p={order} {scheme} {precision}',
+          flush=True)
+    got, _ = _run(backend_factory, 'navier-stokes', n, order, True, scheme,
+                  precision=precision)
+    ref, _ = _run(backend_factory, 'navier-stokes', n, order, False, scheme,
+                  precision=precision)
+    tol = {'double': 1e-14, 'single': 2e-6, 'mixed': 1e-6}[precision]
+    assert rel_l2(got, ref) < tol
+
+
+def test_normals_match_is_checked():
+    """A periodic pair of faces whose vertices differ beyond rounding keeps
+    the gradients at its interfaces."""
+    from pyfr_amd.solvers import NavierStokesIntInters
+    m = BoxMesh(2)
+    el = _Faces(m, 2)
+    i = NavierStokesIntInters.__new__(NavierStokesIntInters)
+    from pyfr_amd.solvers import Interside
+    i.lhs, i.rhs = (Interside(s) for s in m.con)
+    i.elemap, i._perm = {'hex': el}, Ellipsis
+    assert i.normals_match
+    # vertex 0 of element 0 (x = 0 side) moved by 1e-8
+    m.spts['hex'][0, 0, 1] += 1e-8
+    i.elemap = {'hex': _Faces(m, 2)}
+    del i.__dict__['normals_match']
+    assert not i.normals_match
+
+
+class _Faces:
+    """The parts of an element type that its interfaces' normals need."""
+
+    def __init__(self, mesh, order):
+        from pyfr_amd.solvers import FluidElements
+        cfg = make_cfg('euler', order)
+        e = FluidElements(HexShape, mesh.spts['hex'], cfg)
+        self.nfacefpts = e.nfacefpts
+        self.get_pnorms_for_inters = e.get_pnorms_for_inters
