@@ -221,7 +221,9 @@ int frhip_hex_nsvol(void *plan, int geo, int neles, const void *u, long ldu,
  * 64-element block, the flux evaluated once per point into LDS, and (FP32)
  * variant 64: the 4x4x1 MFMA form, 65: the same in blocks of the five
  * wavefronts of an element block (one workgroup, so one XCD's L2 serves
- * every variable's reads of u).  c may be u itself (an RHS in place):
+ * every variable's reads of u), 66: with the operator staged in LDS, each
+ * of the three + 256 s: its rows split over s row groups.  The variants are
+ * timed with an RK4 stage's epilogue.  c may be u itself (an RHS in place):
  * such a call runs variant 32, whose block barriers order every read of u
  * before any write of c, whatever the plan's variant.
  * ep 10..13: RK4 stages 1..4 on four registers, with the update axnpby of

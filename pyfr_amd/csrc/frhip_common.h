@@ -5,6 +5,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <string>
+#include <type_traits>
 
 #include "../../include/frhip.h"
 
@@ -70,6 +71,43 @@ __device__ __forceinline__ unsigned xcd_block()
     const unsigned b = blockIdx.x, nb = gridDim.x;
     const unsigned per = nb/8, rem = nb % 8, x = b % 8;
     return x*per + min(x, rem) + b/8;
+}
+
+// Element row of p at a uniform offset u (elements; scalar registers) plus a
+// lane's byte offset: one 32-bit register addresses all rows of an array.
+template <typename T>
+__device__ __forceinline__ T &at(T *p, long u, unsigned lane)
+{
+    using C = typename std::conditional<std::is_const<T>::value, const char,
+                                        char>::type;
+    return *reinterpret_cast<T *>(reinterpret_cast<C *>(p + u) + lane);
+}
+
+// The same where p and u are uniform in a loop: the row's address is made
+// opaque (scalar), or loop optimisation folds the lane's offset into a
+// 64-bit vector address for every access.
+template <typename T>
+using GlobalRef = T __attribute__((address_space(1))) &;
+
+template <typename T>
+__device__ __forceinline__ GlobalRef<T> row_at(T *p, long u, unsigned lane)
+{
+    const uintptr_t q = reinterpret_cast<uintptr_t>(p + u);
+    const uintptr_t lo = (unsigned)__builtin_amdgcn_readfirstlane((int)q);
+    const uintptr_t hi = (unsigned)__builtin_amdgcn_readfirstlane(
+        (int)(q >> 32));
+    using B = char __attribute__((address_space(1)));
+    using G = T __attribute__((address_space(1)));
+    return *(G *)((B *)(hi << 32 | lo) + lane);
+}
+
+// A pointer read from memory, known to point to device memory (accesses
+// through it are otherwise flat: they also occupy and wait for the LDS path).
+template <typename T>
+__device__ __forceinline__ T *global_ptr(T *p)
+{
+    using G = T __attribute__((address_space(1)));
+    return (T *)(G *)p;
 }
 
 inline hipStream_t as_stream(void *s) { return static_cast<hipStream_t>(s); }

@@ -142,8 +142,8 @@ __device__ __forceinline__ void epi1(T acc, T *__restrict__ c, long off,
             // pointers {r1, r0, dt}, dta the step read from dt once per
             // kernel (rk4_dt); c receives the next stage's input.
             T *const *pp = static_cast<T *const *>(xa);
-            T *r1 = pp[0] + off;
-            const T r0 = pp[1][off];
+            T *r1 = global_ptr(pp[0]) + off;
+            const T r0 = global_ptr(pp[1])[off];
             T n1, nc;
             rk4_vals<T, EP>(t, r0, EP == 10 ? T(0) : *r1, dta, n1, nc);
             *r1 = n1;
@@ -168,7 +168,8 @@ __device__ __forceinline__ void epi1(T acc, T *__restrict__ c, long off,
 // wavefront's accumulators and is split; so is a shorter one where there
 // are too few 64-column groups to fill the chip (the tuner decides).  Each
 // group reads B again, from the L2.  Before, operators past 7 tiles ran on
-// the scalar kernel: 120 x 40 on 726 FP64 prisms took 905 us, now 19 us.
+// the scalar kernel: 120 x 40 on 726 FP64 prisms took 905 us a launch, in
+// row groups 11 to 25.
 template <typename T, int MT, int EP>
 __device__ __forceinline__ void dense_tiles(
     int m, int ks0, int ks1, int k0, int k1, const T *__restrict__ af,
@@ -679,136 +680,246 @@ __device__ __forceinline__ void mfma4x4_chunk(
     (mfma4x4_k<G, KK>(acc, a, b[KK]), ...);
 }
 
-// One wavefront per (64-element block, variable), in blocks of 4 or 5
-// wavefronts (FR_V4 / FR_V4B); no barrier orders the variables' reads of u
-// before another's writes, so c must not alias u (an RHS in place runs the
-// block-cooperative form instead).  Up to 10 row groups (tets p <= 4) the
-// kernel is held to 128 VGPRs, four wavefronts per SIMD: uncapped, the
-// epilogues with 1/|J| take 132-133 and run three (a few spilled registers
-// cost less than the lost wavefront: p = 4 tets, 0.682 -> 0.648 ms per RHS
-// and 6.66 -> 6.09 ms per RK4 step on the 48^3 x 6 box).
-template <int G, int EP>
-__global__ __launch_bounds__(320)
-__attribute__((amdgpu_waves_per_eu(G <= 10 ? 4 : 2))) void k_tdivf_flux4(
-    int m, int nupts, int nc0, int nc1, int k1, const float *__restrict__ af,
-    long ncol, const float *__restrict__ u, long ldu,
-    const float *__restrict__ sm, long lds, const float *__restrict__ b1,
-    long ld1, float *__restrict__ c, long ldc, const float *__restrict__ rcp,
-    long ldr, void *__restrict__ xa, double dta, double dtb, float gm1)
+// One wavefront per (64-element block, variable) and row group of G 4-row
+// groups (blockIdx.y: prisms and pyramids of high order have few element
+// blocks and many rows), in blocks of 4 or 5 wavefronts (FR_V4 / FR_V4B); no
+// barrier orders the variables' reads of u before another's writes, so c
+// must not alias u (an RHS in place runs the block-cooperative form
+// instead).  Up to 10 row groups the kernel is held to four wavefronts per
+// SIMD.
+//
+// Everything that depends on the wavefront is scalar (its element block,
+// its variable, all addresses but the lane's 4 bytes).  Each chunk's
+// operands are requested while the chunk before computes: u right after its
+// flux, the operator right after its MFMAs.  The flux of variable v,
+// transformed, is X/rho (S rho v) + p S e_v with X = rho, rho v_(v-1) or
+// E + p.
+//
+// Bound by memory and the matrix cores in turn: p = 4 pyramids took 90 us,
+// 62 without the reads of u and fn, 44 without the MFMAs.  With the loads of
+// each chunk unconditional the two overlap (p = 4 tets, 35 rows: 55,296 of
+// them 68 -> 57 us, 663,552 604 -> 545; p = 4 pyramids, 55 rows: 34,944 90
+// -> 80 in two row groups, 196,608 509 -> 359 staged).
+//
+// LDSA: the row group's operator is staged in LDS once per block (8
+// wavefronts), four groups of a lane side by side (ds_read_b128), which pays
+// where blocks are many and rows too many for the unstaged form's registers.
+template <int G, int EP, bool LDSA>
+__global__ __launch_bounds__(LDSA ? 512 : 320)
+__attribute__((amdgpu_waves_per_eu(G <= 10 ? 4 : 3))) void k_tdivf_flux4(
+    int m, int nupts, int nc0, int nc1, int k1, int gt,
+    const float *__restrict__ af, long ncol, const float *__restrict__ u,
+    long ldu, const float *__restrict__ sm, long lds,
+    const float *__restrict__ b1, long ld1, float *__restrict__ c, long ldc,
+    const float *__restrict__ rcp, long ldr, void *__restrict__ xa,
+    double dta, double dtb, float gm1)
 {
     dta = rk4_dt<EP>(xa, dta);
-    const int lane = threadIdx.x & 63;
-    const long w = (long)xcd_block()*(blockDim.x >> 6) + (threadIdx.x >> 6);
-    if (w*64 >= ncol) return;
-    const long c0 = w*64;
-    const int v = (int)((c0 >> 6) % 5);
-    const long eb = c0/320, ecol = eb*64 + lane;
+    const unsigned lane = (threadIdx.x & 63)*4;     // byte offset
+    extern __shared__ __attribute__((aligned(16))) char fr_smem[];
+    const float *sa = reinterpret_cast<const float *>(fr_smem);
+    if constexpr (LDSA) {
+        float *sw = reinterpret_cast<float *>(fr_smem);
+        const int g1 = blockIdx.y*G;
+        // one fragment per wavefront and trip (all trip counts uniform)
+        const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        const int l = threadIdx.x & 63;
+        for (int f = wv; f < (nc0 + nc1)*G; f += blockDim.x >> 6) {
+            const int q = f/G, g = f - q*G;
+            const int d = g < G/4*4 ? (g & ~3)*64 + l*4 + (g & 3)
+                                    : g*64 + l;
+            sw[q*G*64 + d] = af[((long)q*gt + g1 + g)*64 + l];
+        }
+        __syncthreads();
+    }
+    // its 32 bits made anew in each basic block: hoisted as a 64-bit value,
+    // no access would use scalar base + lane addressing
+    auto lane32 = [lane]() {
+        unsigned l = lane;
+        asm volatile("" : "+v"(l));
+        return l;
+    };
+    const int w = xcd_block()*(blockDim.x >> 6) +
+                  __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (w*64L >= ncol) return;
+    const long c0 = w*64L;
+    const int v = w % 5;
+    const long eb = w/5, e0 = eb*64;
+    const int g0 = blockIdx.y*G;
 
-    float S[3][3];
+    float S[3][3], Sv[3];
 #pragma unroll
-    for (int i = 0; i < 3; ++i)
+    for (int i = 0; i < 3; ++i) {
 #pragma unroll
-        for (int k = 0; k < 3; ++k) S[i][k] = sm[(3*i + k)*lds + ecol];
+        for (int k = 0; k < 3; ++k) S[i][k] = row_at(sm, (3*i + k)*lds + e0, lane);
+        Sv[i] = v == 1 ? S[i][0] : v == 2 ? S[i][1] : v == 3 ? S[i][2] : 0.0f;
+    }
 
     FrV4f acc[G];
 #pragma unroll
     for (int g = 0; g < G; ++g) acc[g] = FrV4f{0, 0, 0, 0};
 
-    const float *ub = u + eb*320 + lane;
-    const float *afl = af + lane;
-    // u of chunk q + 1 is requested while chunk q computes; points past
-    // the end re-read the last point, whose operator columns are zero
-    float un[5][5];
-#pragma unroll
-    for (int pp = 0; pp < 5; ++pp)
-#pragma unroll
-        for (int x = 0; x < 5; ++x)
-            un[pp][x] = ub[min(pp, nupts - 1)*ldu + x*64];
-    // the operator fragments of chunk q + 1 likewise
-    float an[G];
-#pragma unroll
-    for (int g = 0; g < G; ++g) an[g] = afl[(long)g*64];
-    for (int q = 0; q < nc0; ++q) {
-        float a[G];
-        const long qn = min(q + 1, nc0 + nc1 - 1);
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-            a[g] = an[g];
-            an[g] = afl[(qn*G + g)*64];
-        }
-        float uc[5][5];
-#pragma unroll
-        for (int pp = 0; pp < 5; ++pp)
-#pragma unroll
-            for (int x = 0; x < 5; ++x) {
-                uc[pp][x] = un[pp][x];
-                un[pp][x] = ub[min(5*(q + 1) + pp, nupts - 1)*ldu + x*64];
-            }
-        // this variable's transformed flux at the chunk's 5 points
-        // (flux.mako:3-26, tflux.mako:24-28)
-        float b[15];
+    // points and rows past the end re-read the last one, whose operator
+    // columns are zero
+    const float *ub = u + eb*320, *bb = b1 + c0;
+    float nx[25], a[G];          // the next chunk's u, or fn
+    auto load_u = [&](int q) {
+        const unsigned lane = lane32();
 #pragma unroll
         for (int pp = 0; pp < 5; ++pp) {
-            const float *uw = uc[pp];
-            const float invrho = 1.0f/uw[0], E = uw[4];
-            const float rv[3] = {uw[1], uw[2], uw[3]};
-            const float vel[3] = {invrho*rv[0], invrho*rv[1], invrho*rv[2]};
-            const float p = gm1*(E - 0.5f*invrho*((rv[0])*(rv[0]) +
-                                                  (rv[1])*(rv[1]) +
-                                                  (rv[2])*(rv[2])));
-            float fv[3];
-            if (v == 0) {
-                fv[0] = rv[0]; fv[1] = rv[1]; fv[2] = rv[2];
-            }
-            else if (v == 4) {
-                fv[0] = (E + p)*vel[0]; fv[1] = (E + p)*vel[1];
-                fv[2] = (E + p)*vel[2];
-            }
-            else {
-                const float vj = v == 1 ? vel[0] : v == 2 ? vel[1] : vel[2];
-                fv[0] = v == 1 ? rv[0]*vj + p : rv[0]*vj;
-                fv[1] = v == 2 ? rv[1]*vj + p : rv[1]*vj;
-                fv[2] = v == 3 ? rv[2]*vj + p : rv[2]*vj;
-            }
+            const long r = min(5*q + pp, nupts - 1)*ldu;
 #pragma unroll
-            for (int d = 0; d < 3; ++d)
-                b[3*pp + d] = S[d][0]*fv[0] + S[d][1]*fv[1] + S[d][2]*fv[2];
+            for (int x = 0; x < 5; ++x)
+                nx[5*pp + x] = row_at(ub, r + x*64, lane);
         }
-        mfma4x4_chunk(acc, a, b, std::make_integer_sequence<int, 15>{});
-    }
-
-    // common normal fluxes at the flux points, 16 rows per chunk (rows past
-    // the end re-read the last row; their operator columns are zero)
-    const float *bl = b1 + c0 + lane;
-    for (int q = 0; q < nc1; ++q) {
-        float a[G], b[16];
-        const long qn = min(nc0 + q + 1, nc0 + nc1 - 1);
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-            a[g] = an[g];
-            an[g] = afl[(qn*G + g)*64];
-        }
+    };
+    auto load_b = [&](int q) {
+        const unsigned lane = lane32();
 #pragma unroll
         for (int kk = 0; kk < 16; ++kk)
-            b[kk] = bl[min(16*q + kk, k1 - 1)*ld1];
+            nx[kk] = row_at(bb, min(16*q + kk, k1 - 1)*ld1, lane);
+    };
+    auto load_a = [&](int q) {
+        // after the MFMAs that use a, into the same registers
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (LDSA) {
+            const float *s = sa + min(q, nc0 + nc1 - 1)*G*64;
+            const int l = threadIdx.x & 63;
+#pragma unroll
+            for (int g = 0; g < G/4; ++g) {
+                const FrV4f t = *reinterpret_cast<const FrV4f *>(
+                    s + g*256 + l*4);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) a[4*g + i] = t[i];
+            }
+#pragma unroll
+            for (int g = G/4*4; g < G; ++g) a[g] = s[g*64 + l];
+            return;
+        }
+        const unsigned lane = lane32();
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+            a[g] = row_at(af, ((long)q*gt + g0)*64, lane + g*256);
+    };
+    // this variable's transformed flux at the chunk's 5 points (flux.mako:
+    // 3-26, tflux.mako:24-28); frees nx for the next request
+    auto flux = [&](float (&b)[15]) {
+#pragma unroll
+        for (int pp = 0; pp < 5; ++pp) {
+            const float *uw = nx + 5*pp;
+            const float invrho = 1.0f/uw[0];
+            const float rv[3] = {uw[1], uw[2], uw[3]};
+            const float p = gm1*(uw[4] - 0.5f*invrho*((rv[0])*(rv[0]) +
+                                                      (rv[1])*(rv[1]) +
+                                                      (rv[2])*(rv[2])));
+            // selected after it is computed, or branches on v come back
+            float y = uw[4] + p;
+            asm volatile("" : "+v"(y));
+            y = v == 1 ? rv[0] : v == 2 ? rv[1] : v == 3 ? rv[2] : y;
+            float x = invrho*y;
+            asm volatile("" : "+v"(x));
+            x = v == 0 ? 1.0f : x;
+#pragma unroll
+            for (int d = 0; d < 3; ++d)
+                b[3*pp + d] = x*(S[d][0]*rv[0] + S[d][1]*rv[1] +
+                                 S[d][2]*rv[2]) + p*Sv[d];
+        }
+#pragma unroll
+        for (int k = 0; k < 15; ++k) asm volatile("" : "+v"(b[k]));
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // No branch decides what is requested: where a path with fewer requests
+    // in flight joins, the wait for the operator covers part of the u
+    // requested after it, and every chunk's MFMAs wait for the next u.
+    load_u(0);
+    load_a(0);
+#pragma unroll 1
+    for (int q = 0; q < nc0 - 1; ++q) {
+        float b[15];
+        flux(b);
+        load_u(q + 1);
+        mfma4x4_chunk(acc, a, b, std::make_integer_sequence<int, 15>{});
+        load_a(q + 1);
+    }
+    {
+        float b[15];
+        flux(b);
+        load_b(0);
+        mfma4x4_chunk(acc, a, b, std::make_integer_sequence<int, 15>{});
+        load_a(nc0);
+    }
+    // common normal fluxes at the flux points, 16 rows per chunk (the last
+    // chunk is requested once more than it is used)
+#pragma unroll 1
+    for (int q = 0; q < nc1; ++q) {
+        float b[16];
+#pragma unroll
+        for (int kk = 0; kk < 16; ++kk) b[kk] = nx[kk];
+        load_b(q + 1);
         mfma4x4_chunk(acc, a, b, std::make_integer_sequence<int, 16>{});
+        load_a(min(nc0 + q + 1, nc0 + nc1 - 1));
     }
 
-#pragma unroll
-    for (int g = 0; g < G; ++g)
+    // Epilogue.  The RK stages' registers are read one 4-row group ahead of
+    // the stores, which the compiler cannot move loads across: row by row,
+    // each waited for memory in turn (75 rows of prisms: 119-160 us a stage
+    // against 66 for the plain store).
+    constexpr bool RK = EP == 2 || EP == 4 || EP >= 10;
+    constexpr bool R0 = EP >= 10 && EP != 13, R1 = RK && EP != 10;
+    float *r1 = nullptr;
+    const float *r0 = nullptr;
+    if constexpr (EP >= 10) {
+        r1 = global_ptr(static_cast<float *const *>(xa)[0]);
+        r0 = global_ptr(static_cast<float *const *>(xa)[1]);
+    }
+    else if constexpr (RK)
+        r1 = static_cast<float *>(xa);
+    float x1[2][4] = {}, x0[2][4] = {}, rc[2][4] = {};
+    auto load_rk = [&](int g) {
+        const unsigned lane = lane32();
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int row = 4*g + i;
-            if (row >= m) continue;
-            const long off = row*ldc + c0 + lane;
-            if constexpr (EP == 0)
-                c[off] = acc[g][i];
-            else if constexpr (EP == 1)
-                c[off] = -rcp[row*ldr + ecol]*acc[g][i];
-            else
-                epi1<float, EP>(acc[g][i], c, off, rcp, row*ldr + ecol,
-                                xa, dta, dtb, 1.0f, 0.0f);
+            const long row = min(4*(g0 + g) + i, m - 1);
+            if constexpr (EP != 0)
+                rc[g & 1][i] = row_at(rcp, row*ldr + e0, lane);
+            if constexpr (R1) x1[g & 1][i] = row_at(r1, row*ldc + c0, lane);
+            if constexpr (R0) x0[g & 1][i] = row_at(r0, row*ldc + c0, lane);
         }
+    };
+    load_rk(0);
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        if (g + 1 < G) load_rk(g + 1);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int row = 4*(g0 + g) + i;
+            if (row >= m) continue;
+            const unsigned lane = lane32();
+            const long off = row*ldc + c0;
+            const float t = EP == 0 ? acc[g][i] : -rc[g & 1][i]*acc[g][i];
+            const float y1 = x1[g & 1][i], y0 = x0[g & 1][i];
+            (void)y1; (void)y0;
+            if constexpr (EP <= 1)
+                row_at(c, off, lane) = t;
+            else if constexpr (EP == 2) {
+                row_at(r1, off, lane) = y1 + float(dta)*t;
+                row_at(c, off, lane) = y1 + float(dtb)*t;
+            }
+            else if constexpr (EP == 4)
+                row_at(r1, off, lane) = y1 + float(dtb)*t;
+            else if constexpr (EP >= 10) {
+                float n1, nc;
+                rk4_vals<float, EP>(t, y0, y1, dta, n1, nc);
+                row_at(r1, off, lane) = n1;
+                if constexpr (EP != 13) row_at(c, off, lane) = nc;
+            }
+            else
+                epi1<float, EP>(acc[g][i], c, off + lane/4, rcp,
+                                row*ldr + e0 + lane/4, xa, dta, dtb, 1.0f,
+                                0.0f);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
 }
 
 // ---- dispatch -------------------------------------------------------------
@@ -827,6 +938,10 @@ constexpr int FR_V4 = 64;
 // variables in one workgroup, so on one XCD and its L2: u is fetched from
 // HBM once, not once per XCD the variables land on)
 constexpr int FR_V4B = 65;
+// ... with the operator staged in LDS, eight wavefronts per block
+constexpr int FR_V4L = 66;
+// any of the three + 256 s: the 4-row groups split over s row groups
+constexpr int FR_G4MAX = 10;    // 4-row groups of an unstaged wavefront
 constexpr size_t FR_LDS_MAX = 65536;
 
 // Row tiles one wavefront's accumulators hold
@@ -1307,6 +1422,35 @@ static bool flux4_ok(int g)
            g == 9 || g == 10 || g == 14 || g == 19;
 }
 
+static bool is_flux4(int v)
+{
+    const int b = v % FR_SPLIT;
+    return b == FR_V4 || b == FR_V4B || b == FR_V4L;
+}
+
+// 4-row groups per wavefront of variant v: the smallest instantiation that
+// covers a split into v/FR_SPLIT row groups.  The unstaged form holds at
+// most FR_G4MAX (with more it keeps the operator's addresses and loads in
+// flight in scratch memory) and splits further by itself.
+static int flux4_group(int gt, int v)
+{
+    int s = std::max(v/FR_SPLIT, 1);
+    if (v % FR_SPLIT != FR_V4L) s = std::max(s, (gt + FR_G4MAX - 1)/FR_G4MAX);
+    int g = (gt + s - 1)/s;
+    while (g != 7 && !flux4_ok(g)) ++g;
+    return g;
+}
+
+// LDS of the staged form: nc chunks of gw 4-row groups
+static size_t flux4_lds(int nc, int gw) { return (size_t)nc*gw*64*4; }
+
+static bool flux4_valid(int v, int gt, int nc)
+{
+    return v >= 0 && v/FR_SPLIT <= gt &&
+           (v % FR_SPLIT != FR_V4L ||
+            flux4_lds(nc, flux4_group(gt, v)) <= FR_LDS_MAX);
+}
+
 template <typename T, int EP>
 static void launch_flux_ep(const FluxPlan *p, int wpb, long ncol,
                            const void *u, long ldu, const void *sm, long lds,
@@ -1315,22 +1459,31 @@ static void launch_flux_ep(const FluxPlan *p, int wpb, long ncol,
                            double dtb, double gamma, hipStream_t s)
 {
     if constexpr (sizeof(T) == 4) {
-        if (wpb == FR_V4 || wpb == FR_V4B) {
-            const int wv = wpb == FR_V4B ? 5 : 4;
-            const dim3 grid(cdiv(ncol/64, wv)), block(64*wv);
+        if (is_flux4(wpb)) {
+            const bool ldsa = wpb % FR_SPLIT == FR_V4L;
+            const int wv = ldsa ? 8 : wpb % FR_SPLIT == FR_V4B ? 5 : 4;
+            const int gw = flux4_group(p->g4, wpb);
+            const size_t smem = ldsa ? flux4_lds(p->nc0 + p->nc1, gw) : 0;
+            const dim3 grid(cdiv(ncol/64, wv), cdiv(p->g4, gw));
+            const dim3 block(64*wv);
 #define FR_G4(GV)                                                           \
-            case GV:                                                        \
-                hipLaunchKernelGGL((k_tdivf_flux4<GV, EP>), grid, block, 0, \
+            case GV: {                                                      \
+                auto k = k_tdivf_flux4<GV, EP, true>;                       \
+                if constexpr (GV <= FR_G4MAX)                               \
+                    if (!ldsa) k = k_tdivf_flux4<GV, EP, false>;            \
+                hipLaunchKernelGGL(k, grid, block, smem,                    \
                                    s, p->d.m, p->nupts, p->nc0, p->nc1,     \
-                                   p->d.k1, (const float *)p->af4, ncol,    \
+                                   p->d.k1, p->g4, (const float *)p->af4,   \
+                                   ncol,                                    \
                                    (const float *)u, ldu, (const float *)sm,\
                                    lds, (const float *)fn, ldf, (float *)c, \
                                    ldc, (const float *)rcp, ldr, xa, dta,   \
                                    dtb, (float)(gamma - 1));                \
-                break;
-            switch (p->g4) {
-                FR_G4(1) FR_G4(2) FR_G4(3) FR_G4(4) FR_G4(5) FR_G4(8)
-                FR_G4(9) FR_G4(10) FR_G4(14) FR_G4(19)
+                break;                                                      \
+            }
+            switch (gw) {
+                FR_G4(1) FR_G4(2) FR_G4(3) FR_G4(4) FR_G4(5) FR_G4(7)
+                FR_G4(8) FR_G4(9) FR_G4(10) FR_G4(14) FR_G4(19)
             }
 #undef FR_G4
             return;
@@ -1433,9 +1586,10 @@ static int flux_launch(const FluxPlan *p, int ep, long ncol, const void *u,
     FR_CHECK(ep < 2 || xa, "RK epilogue needs the r1 / accumulator array");
     const size_t esz = p->d.dtype == FRHIP_F64 ? 8 : 4;
     int wpb = p->d.variant > 0 ? p->d.variant : 4;
-    if ((wpb == FR_V4 || wpb == FR_V4B) && !p->af4)
+    if (is_flux4(wpb) && (!p->af4 ||
+                          !flux4_valid(wpb, p->g4, p->nc0 + p->nc1)))
         wpb = 4;
-    if (wpb != FR_BLKV && wpb != FR_V4 && wpb != FR_V4B &&
+    if (wpb != FR_BLKV && !is_flux4(wpb) &&
         !variant_valid(wpb, (size_t)p->d.mt*(p->d.ks0 + p->d.ks1)*64*esz,
                        false))
         wpb &= ~FR_LDSV;
@@ -1511,7 +1665,9 @@ int frhip_tdivf_plan_create(void **plan, int m, int nupts, int nfpts,
     void *d4 = nullptr;
     const int g4 = (m + 3)/4, nc0 = (nupts + 4)/5, nc1 = (nfpts + 15)/16;
     if (dtype == FRHIP_F32 && flux4_ok(g4)) {
-        std::vector<float> f4((size_t)(nc0 + nc1)*g4*64, 0.0f);
+        // a split's last row group and the last chunk's prefetch may run
+        // past the operator
+        std::vector<float> f4((size_t)((nc0 + nc1 + 1)*g4 + 32)*64, 0.0f);
         for (int q = 0; q < nc0 + nc1; ++q)
             for (int g = 0; g < g4; ++g)
                 for (int l = 0; l < 64; ++l) {
@@ -1586,26 +1742,64 @@ int frhip_tdivf_plan_tune(void *plan, int ncol, const void *u, long ldu,
     FluxPlan *p = static_cast<FluxPlan *>(plan);
     FR_CHECK(p && reps > 0, "invalid arguments");
     const size_t esz = p->d.dtype == FRHIP_F64 ? 8 : 4;
-    void *c = nullptr;
-    FR_HIP(hipMalloc(&c, (size_t)p->d.m*ncol*esz));
+    // Timed with an RK4 stage's epilogue (10 + 1: both registers read and
+    // written) on scratch registers, as time steps run the kernel: the plain
+    // store ranks the variants differently (p = 4 prisms, 9,216 of them: 63
+    // us for the 16-row tiles with it, 150 with the epilogue).
+    if (ncol == 0) {
+        if (variant) *variant = p->d.variant;
+        return 0;
+    }
+    const size_t nb = ((size_t)p->d.m*ncol*esz + 255)/256*256;
+    char *scratch = nullptr;
+    FR_HIP(hipMalloc(&scratch, 3*nb + (size_t)ncol*esz + 256));
+    void *c = scratch, *rcp = scratch + 3*nb + 256;
+    char *xa = scratch + 3*nb;
+    void *const ptrs[4] = {scratch + nb, scratch + 2*nb, xa + 24, nullptr};
+    if (hipMemset(scratch, 0, 3*nb + (size_t)ncol*esz + 256) != hipSuccess ||
+        hipMemcpy(xa, ptrs, sizeof(ptrs), hipMemcpyHostToDevice) !=
+            hipSuccess) {
+        (void)hipFree(scratch);
+        set_error("tuning scratch");
+        return 1;
+    }
     hipEvent_t e0, e1;
     (void)hipEventCreate(&e0);
     (void)hipEventCreate(&e1);
     float best = 1e30f;
     int bestv = 4, rc = 0;
     const size_t ldsb = (size_t)p->d.mt*(p->d.ks0 + p->d.ks1)*64*esz;
-    for (int v : {1, 2, 4, FR_LDSV + 1, FR_LDSV + 2, FR_LDSV + 4,
-                  FR_BLKV, FR_V4, FR_V4B}) {
-        if (v == FR_V4 || v == FR_V4B
-                ? !p->af4
+    std::vector<int> cands = {1, 2, 4, FR_LDSV + 1, FR_LDSV + 2, FR_LDSV + 4,
+                              FR_BLKV, FR_V4, FR_V4B, FR_V4L};
+    // A split repeats the flux in every row group: only while the grid is
+    // short of four wavefronts per SIMD (p = 4 pyramids, 34,944 of them: 80
+    // us in two row groups, 98 in one; 196,608: 390 and 359).
+    int last = p->g4;
+    for (int s = 2; s <= p->g4; ++s) {
+        const int gw = flux4_group(p->g4, s*FR_SPLIT + FR_V4L);
+        if (gw == last) continue;
+        if (ncol/64*cdiv(p->g4, last) >= 4096) break;
+        last = gw;
+        cands.push_back(s*FR_SPLIT + FR_V4);
+        cands.push_back(s*FR_SPLIT + FR_V4L);
+    }
+    // the staged form of the smallest split whose operator fits in LDS
+    for (int s = 2; s <= p->g4; ++s)
+        if (flux4_valid(s*FR_SPLIT + FR_V4L, p->g4, p->nc0 + p->nc1)) {
+            cands.push_back(s*FR_SPLIT + FR_V4L);
+            break;
+        }
+    for (int v : cands) {
+        if (is_flux4(v)
+                ? !p->af4 || !flux4_valid(v, p->g4, p->nc0 + p->nc1)
                 : v != FR_BLKV && !variant_valid(v, ldsb, false))
             continue;
         FluxPlan q = *p;
         q.d.variant = v;
         for (int it = 0; it < reps + 1 && !rc; ++it) {
             if (it == 1) (void)hipEventRecord(e0, nullptr);
-            rc = flux_launch(&q, 0, ncol, u, ldu, smats, lds, fn, ldf, c,
-                             ncol, nullptr, 0, nullptr, 0, 0, gamma, nullptr);
+            rc = flux_launch(&q, 11, ncol, u, ldu, smats, lds, fn, ldf, c,
+                             ncol, rcp, 0, xa, 0, 0, gamma, nullptr);
         }
         if (rc) break;
         (void)hipEventRecord(e1, nullptr);
@@ -1619,7 +1813,7 @@ int frhip_tdivf_plan_tune(void *plan, int ncol, const void *u, long ldu,
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    (void)hipFree(c);
+    (void)hipFree(scratch);
     if (rc) return rc;
     p->d.variant = bestv;
     if (variant) *variant = bestv;
@@ -1634,7 +1828,8 @@ int frhip_tdivf_plan_set_variant(void *plan, int variant)
     FR_CHECK(p, "null plan");
     const size_t esz = p->d.dtype == FRHIP_F64 ? 8 : 4;
     FR_CHECK(variant == FR_BLKV ||
-             ((variant == FR_V4 || variant == FR_V4B) && p->af4) ||
+             (is_flux4(variant) && p->af4 &&
+              flux4_valid(variant, p->g4, p->nc0 + p->nc1)) ||
              variant_valid(variant,
                            (size_t)p->d.mt*(p->d.ks0 + p->d.ks1)*64*esz,
                            false), "invalid variant");

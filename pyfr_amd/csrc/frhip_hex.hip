@@ -89,16 +89,6 @@ __device__ __forceinline__ void layer_end(T (&x)[M])
     __builtin_amdgcn_sched_barrier(0);
 }
 
-// Element row of p at a uniform offset u (elements; scalar registers) plus a
-// lane's byte offset: one 32-bit register addresses all rows of an array.
-template <typename T>
-__device__ __forceinline__ T &at(T *p, long u, unsigned lane)
-{
-    using C = typename std::conditional<std::is_const<T>::value, const char,
-                                        char>::type;
-    return *reinterpret_cast<T *>(reinterpret_cast<C *>(p + u) + lane);
-}
-
 // The thread's pencil; uniform (scalar registers) where a wavefront is one
 // pencil of 64 elements.
 template <int EB>
@@ -250,8 +240,8 @@ __device__ __forceinline__ void hex_stage(const HexDivArgs<T> &a, long u,
         // RK4 (steppers.py:67-108), in T or, for the precision form, FP64
         using R = typename std::conditional<FAM == HEX_RK4, T, double>::type;
         R *const *pp = static_cast<R *const *>(a.xa);
-        R *r1 = pp[0];
-        const R *r0 = pp[1];
+        R *r1 = global_ptr(pp[0]);
+        const R *r0 = global_ptr(pp[1]);
         const unsigned orr = off*(unsigned)sizeof(R);
         const int stage = FAM == HEX_RK4 ? a.ep - 9 : a.ep - 13;
         R x[5], y[5];

@@ -201,6 +201,13 @@ def test_pyramid_fp32_flux_variants(backend_factory, variant):
         del integ, sysm
 
 
+@pytest.mark.parametrize('variant', [66, 66 + 2*256])
+def test_pyramid_fp32_staged_flux(backend_factory, variant):
+    """The 4x4x1 MFMA form with the operator staged in LDS, whole (2, 4, 8
+    and 14 4-row groups) and in two row groups."""
+    test_pyramid_fp32_flux_variants(backend_factory, variant)
+
+
 @pytest.mark.parametrize('layout,precision', [('hex-pyr', 'double'),
                                               ('tet-pyt', 'double'),
                                               ('pyr', 'single')])

@@ -288,6 +288,16 @@ def test_flux_variants_parity(backend_factory, precision, variant):
         del integ, sysm
 
 
+@pytest.mark.parametrize('variant', [64 + 2*256, 66 + 2*256, 66 + 3*256])
+def test_flux4_row_splits(backend_factory, variant):
+    """The 4x4x1 MFMA form with its row groups split (+ 256 s) and with the
+    operator staged in LDS (66): 20, 35, 40 and 75 rows in groups that end
+    inside and past the operator, the right-hand side and the RK4 stages,
+    to the bounds of the unsplit form."""
+    test_flux_variants_parity(backend_factory, 'single', variant)
+    test_simplex_rk4_fused_stages(backend_factory, 'single', variant, 4)
+
+
 def test_simplex_rk4_trajectory(backend_factory):
     be = backend_factory()
     integ, orc, u0 = _mixed(be, 3, 2, 1, 3, dt=2e-3)
