@@ -102,6 +102,11 @@ int frhip_graph_destroy(void *graph_exec);
 int frhip_mul_plan_create(void **plan, int m, int k, const double *a_host,
                           int dtype, int *kind);
 int frhip_mul_plan_destroy(void *plan);
+/* C_i = A @ B_i for n pairs of row slabs (B_i = b + i*sb, C_i = c + i*sc, in
+ * elements), as n calls of frhip_mul in order; on the matrix cores in one
+ * launch. */
+int frhip_mul_slabs(void *plan, int n, int ncol, const void *b, long ldb,
+                    long sb, void *c, long ldc, long sc, void *stream);
 int frhip_mul(void *plan, int ncol, const void *b, long ldb, void *c,
               long ldc, double alpha, double beta, void *stream);
 

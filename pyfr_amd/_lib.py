@@ -52,6 +52,7 @@ _FUNCS = {
     'frhip_mul_plan_destroy': [_P],
     'frhip_mul_plan_tune': [_P, _I, _P, _L, _I, ct.POINTER(_I)],
     'frhip_mul': [_P, _I, _P, _L, _P, _L, _D, _D, _P],
+    'frhip_mul_slabs': [_P, _I, _I, _P, _L, _L, _P, _L, _L, _P],
     'frhip_mul2_plan_create': [ct.POINTER(_P), _I, _I, _I, _P, _P, _I,
                                ct.POINTER(_I)],
     'frhip_mul2_plan_destroy': [_P],

@@ -678,6 +678,28 @@ class MulProvider:
         k.kind = {1: 'structured', 2: 'dense', 3: 'bf16'}[kind]
         return k
 
+    def mul_slabs(self, a, b, out, n):
+        """out_i = a b_i for the n row slabs of b and out, as n mul kernels
+        over the slabs would; on the matrix cores in one launch."""
+        if 'const' not in a.tags:
+            raise NotSuitableError('mul requires a constant operator')
+        if n*a.ncol != b.nrow or n*a.nrow != out.nrow:
+            raise ValueError('Incompatible matrices for out = a*b')
+        if b.ncol != out.ncol or b.dtype != out.dtype:
+            raise ValueError('Incompatible matrices for out = a*b')
+        lib = self.backend.lib
+        plan, kind = self._plan(a, b.dtype)
+        ncol, ldb, ldc = b.ncol, b.leaddim, out.leaddim
+        bp, cp = b.data, out.data
+        sb, sc = a.ncol*ldb, a.nrow*ldc
+        if kind == 2:
+            self._tune(lib.mul_plan_tune, plan, ncol, bp, ldb)
+        k = Kernel(lambda stream: lib.mul_slabs(plan, n, ncol, bp, ldb, sb,
+                                                cp, ldc, sc, stream),
+                   mats=(a, b, out), name='mul_slabs')
+        k.kind = {1: 'structured', 2: 'dense', 3: 'bf16'}[kind]
+        return k
+
     # -- fused two-operator applications (no reference counterpart: they fuse
     #    kernels the reference runs back to back, see include/frhip.h)
     def _plan2(self, a0, a1, dtype):

@@ -34,6 +34,16 @@ int dense_plan_create(DensePlan **out, int m, int k0, int k1,
 void dense_plan_destroy(DensePlan *p);
 bool dense_variant_ok(const DensePlan *p, int variant);
 
+// n row slabs of b0 and of c, b and c elements apart, that one launch covers:
+// the three directions of a gradient's interpolation, 5-10 us each on small
+// meshes and bound by latency and launch (a Navier-Stokes step of 11^3 x 8
+// tets and prisms, p = 3, FP64: 774 us with a launch each, 710 with one; of
+// 9^3 x 6 tets, p = 2, FP32, RK4: 180 and 163 us)
+struct Slabs {
+    int n = 1;
+    long b = 0, c = 0;
+};
+
 // ep: 0 store, 1 negdivconf, 2/4 RK45 stage / last stage, 3/5 mixed RK45
 // stage / last stage, 6 c += acc, 7 c = alpha*acc + beta*c, 8 c = alpha*acc.
 // Column j of a 5-variable AoSoA array belongs to element
@@ -42,7 +52,8 @@ bool dense_variant_ok(const DensePlan *p, int variant);
 int dense_launch(const DensePlan *p, int ep, long ncol, const void *b0,
                  long ld0, const void *b1, long ld1, void *c, long ldc,
                  const void *rcp, long ldr, int nvar, void *xa, double dta,
-                 double dtb, double alpha, double beta, hipStream_t s);
+                 double dtb, double alpha, double beta, hipStream_t s,
+                 Slabs sl = {});
 
 // Time the variants on the given inputs (into a scratch output) and keep
 // the fastest.  Synchronous; the inputs must be ready.

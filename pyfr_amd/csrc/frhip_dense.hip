@@ -288,10 +288,12 @@ __global__ __launch_bounds__(256) void k_dense_mfma(
     long ncol, const T *__restrict__ b0, long ld0, const T *__restrict__ b1,
     long ld1, T *__restrict__ c, long ldc, const T *__restrict__ rcp,
     long ldr, int nvar, void *__restrict__ xa, double dta, double dtb,
-    T alpha, T beta)
+    T alpha, T beta, long sb, long sc)
 {
     const long nf = (long)MT*(ks0 + ks1)*64;
     af += blockIdx.y*nf;
+    b0 += blockIdx.z*sb;
+    c += blockIdx.z*sc;
     const T *a = LDSA ? stage_frags(af, (int)nf) : af;
     dense_tiles<T, MT, EP>(m, ks0, ks1, k0, k1, a, ncol, b0, ld0, b1, ld1, c,
                            ldc, rcp, ldr, nvar, xa, dta, dtb, alpha, beta);
@@ -980,7 +982,7 @@ static int launch_ep(const DensePlan *p, int variant, long ncol,
                      const void *b0, long ld0, const void *b1, long ld1,
                      void *c, long ldc, const void *rcp, long ldr, int nvar,
                      void *xa, double dta, double dtb, double alpha,
-                     double beta, hipStream_t s)
+                     double beta, hipStream_t s, Slabs sl)
 {
     const T *pb0 = (const T *)b0, *pb1 = (const T *)b1;
     const T *prcp = (const T *)rcp;
@@ -1001,11 +1003,11 @@ static int launch_ep(const DensePlan *p, int variant, long ncol,
     case MTV: {                                                             \
         auto k = lds ? k_dense_mfma<T, MTV, EP, true>                       \
                      : k_dense_mfma<T, MTV, EP, false>;                     \
-        dim3 grid(cdiv(ncol/64, wpb), cdiv(p->mt, MTV));                    \
+        dim3 grid(cdiv(ncol/64, wpb), cdiv(p->mt, MTV), sl.n);              \
         hipLaunchKernelGGL(k, grid, block, ldsb, s, p->m, p->ks0, p->ks1,   \
                            p->k0, p->k1, (const T *)p->afrag, ncol, pb0,    \
                            ld0, pb1, ld1, (T *)c, ldc, prcp, ldr, nvar, xa, \
-                           dta, dtb, (T)alpha, (T)beta);                    \
+                           dta, dtb, (T)alpha, (T)beta, sl.b, sl.c);        \
         return 0;                                                           \
     }
     switch (mtg) {
@@ -1021,12 +1023,13 @@ static int launch_t(const DensePlan *p, int variant, int ep, long ncol,
                     const void *b0, long ld0, const void *b1, long ld1,
                     void *c, long ldc, const void *rcp, long ldr, int nvar,
                     void *xa, double dta, double dtb, double alpha,
-                    double beta, hipStream_t s)
+                    double beta, hipStream_t s, Slabs sl)
 {
 #define FR_EP(E)                                                            \
     case E:                                                                 \
         return launch_ep<T, E>(p, variant, ncol, b0, ld0, b1, ld1, c, ldc,  \
-                               rcp, ldr, nvar, xa, dta, dtb, alpha, beta, s);
+                               rcp, ldr, nvar, xa, dta, dtb, alpha, beta, s,\
+                               sl);
     switch (ep) {
         FR_EP(0) FR_EP(1) FR_EP(2) FR_EP(4) FR_EP(6) FR_EP(7) FR_EP(8)
         case 3: case 5:
@@ -1034,10 +1037,10 @@ static int launch_t(const DensePlan *p, int variant, int ep, long ncol,
                 if (ep == 3)
                     return launch_ep<T, 3>(p, variant, ncol, b0, ld0, b1,
                                            ld1, c, ldc, rcp, ldr, nvar, xa,
-                                           dta, dtb, alpha, beta, s);
+                                           dta, dtb, alpha, beta, s, sl);
                 return launch_ep<T, 5>(p, variant, ncol, b0, ld0, b1, ld1,
                                        c, ldc, rcp, ldr, nvar, xa, dta, dtb,
-                                       alpha, beta, s);
+                                       alpha, beta, s, sl);
             }
             break;
     }
@@ -1129,16 +1132,35 @@ void dense_plan_destroy(DensePlan *p)
 int dense_launch(const DensePlan *p, int ep, long ncol, const void *b0,
                  long ld0, const void *b1, long ld1, void *c, long ldc,
                  const void *rcp, long ldr, int nvar, void *xa, double dta,
-                 double dtb, double alpha, double beta, hipStream_t s)
+                 double dtb, double alpha, double beta, hipStream_t s,
+                 Slabs sl)
 {
     int variant = p->variant;
     if (variant != 0 && !mfma_ok(p, ncol, b0, ld0, b1, ld1, c, ldc))
         variant = 0;
     if (!dense_valid(p, variant))
         variant &= ~FR_LDSV;
+    const size_t esz = p->dtype == FRHIP_F64 ? 8 : 4;
+    // slabs in one launch: matrix cores only, starts as aligned as the
+    // first, and no slab's output may be another's input
+    if (sl.n > 1) {
+        const uintptr_t bp = (uintptr_t)b0, cp = (uintptr_t)c;
+        const size_t be = ((sl.n - 1)*sl.b + (p->k0 - 1)*ld0 + ncol)*esz,
+                     ce = ((sl.n - 1)*sl.c + (p->m - 1)*ldc + ncol)*esz;
+        if (variant == 0 || sl.b % 4 || sl.c % 4 ||
+            sl.c < (p->m - 1)*ldc + ncol || (bp < cp + ce && cp < bp + be)) {
+            for (int i = 0; i < sl.n; ++i) {
+                const int rc = dense_launch(
+                    p, ep, ncol, (const char *)b0 + i*sl.b*esz, ld0, b1, ld1,
+                    (char *)c + i*sl.c*esz, ldc, rcp, ldr, nvar, xa, dta,
+                    dtb, alpha, beta, s);
+                if (rc) return rc;
+            }
+            return 0;
+        }
+    }
     // in place, each column's reads of B must precede its writes: one
     // wavefront for all rows
-    const size_t esz = p->dtype == FRHIP_F64 ? 8 : 4;
     auto meets = [&](const void *b, int k, long ld) {
         const uintptr_t b0p = (uintptr_t)b, cp = (uintptr_t)c;
         return b && b0p < cp + ((p->m - 1)*ldc + ncol)*esz &&
@@ -1149,9 +1171,9 @@ int dense_launch(const DensePlan *p, int ep, long ncol, const void *b0,
         variant %= FR_SPLIT;
     const int rc = p->dtype == FRHIP_F64
         ? launch_t<double>(p, variant, ep, ncol, b0, ld0, b1, ld1, c, ldc,
-                           rcp, ldr, nvar, xa, dta, dtb, alpha, beta, s)
+                           rcp, ldr, nvar, xa, dta, dtb, alpha, beta, s, sl)
         : launch_t<float>(p, variant, ep, ncol, b0, ld0, b1, ld1, c, ldc,
-                          rcp, ldr, nvar, xa, dta, dtb, alpha, beta, s);
+                          rcp, ldr, nvar, xa, dta, dtb, alpha, beta, s, sl);
     if (rc) return rc;
     FR_LAUNCHED();
     return 0;

@@ -132,6 +132,31 @@ int frhip_mul_plan_destroy(void *plan)
     FR_API_END
 }
 
+int frhip_mul_slabs(void *plan, int n, int ncol, const void *b, long ldb,
+                    long sb, void *c, long ldc, long sc, void *stream)
+{
+    FR_API_BEGIN
+    MulPlan *p = static_cast<MulPlan *>(plan);
+    FR_CHECK(p, "null plan");
+    FR_CHECK(n >= 0 && n <= 65535 && sb >= 0 && sc >= 0,
+             "invalid mul slabs");
+    FR_CHECK(ncol >= 0 && ldb >= ncol && ldc >= ncol, "invalid mul extents");
+    if (ncol == 0 || n == 0) return 0;
+    if (p->kind == 2)
+        return dense_launch(p->dense, 0, ncol, b, ldb, nullptr, 0, c, ldc,
+                            nullptr, 0, 1, nullptr, 0, 0, 1.0, 0.0,
+                            as_stream(stream), {n, sb, sc});
+    const long esz = p->dtype == FRHIP_F64 ? 8 : 4;
+    for (int i = 0; i < n; ++i) {
+        const int rc = frhip_mul(p, ncol, (const char *)b + i*sb*esz, ldb,
+                                 (char *)c + i*sc*esz, ldc, 1.0, 0.0,
+                                 stream);
+        if (rc) return rc;
+    }
+    return 0;
+    FR_API_END
+}
+
 int frhip_mul(void *plan, int ncol, const void *b, long ldb, void *c,
               long ldc, double alpha, double beta, void *stream)
 {

@@ -695,15 +695,9 @@ class NavierStokesElements(EulerElements):
             beta=float(self.basis.order > 0))
 
         # pyfr/solvers/baseadvecdiff/elements.py:87-101
-        def gradcoru_fpts():
-            nupts, nfpts = self.nupts, self.nfpts
-            vu, vf = self._grad_upts, self._vect_fpts
-            muls = [be.kernel('mul', self.opmat('M0'),
-                              vu.slice(i*nupts, (i + 1)*nupts),
-                              vf.slice(i*nfpts, (i + 1)*nfpts))
-                    for i in range(self.ndims)]
-            return be.unordered_meta_kernel(muls)
-        kernels['gradcoru_fpts'] = gradcoru_fpts
+        kernels['gradcoru_fpts'] = lambda: be.kernel(
+            'mul_slabs', self.opmat('M0'), self._grad_upts, self._vect_fpts,
+            self.ndims)
 
         # pyfr/solvers/navstokes/elements.py:31-128 (tdisf_fused)
         visc_corr = self.cfg.get('solver', 'viscosity-correction', 'none')

@@ -142,6 +142,39 @@ def test_dense_row_groups(backend_factory, precision, variant, shape):
 
 
 @pytest.mark.parametrize('precision', ['double', 'single'])
+@pytest.mark.parametrize('variant', [0, 1, 17, 2*256 + 1])
+@pytest.mark.parametrize('m,k,neles', [(40, 20, 70), (18, 10, 1),
+                                       (33, 35, 200)])
+def test_mul_slabs(backend_factory, precision, variant, m, k, neles):
+    """One operator over three row slabs in one call against a call per
+    slab: the same bytes, on the matrix cores and with the scalar kernel."""
+    from pyfr_amd.backend import MulProvider
+    be = backend_factory(precision=precision)
+    rng = np.random.default_rng(m)
+    a = be.const_matrix(rng.standard_normal((m, k)))
+    b = be.matrix((3*k, 5, neles), rng.standard_normal((3*k, 5, neles)),
+                  tags={'align'})
+    c, d = (be.matrix((3*m, 5, neles),
+                      rng.standard_normal((3*m, 5, neles)), tags={'align'})
+            for _ in range(2))
+    print(f'\n[mul slabs] {precision} {m}x{k} v={variant}', flush=True)
+    one = be.kernel('mul_slabs', a, b, c, 3)
+    sep = [be.kernel('mul', a, b.slice(i*k, (i + 1)*k),
+                     d.slice(i*m, (i + 1)*m)) for i in range(3)]
+    mp = next(p for p in be._providers if isinstance(p, MulProvider))
+    be.lib.mul_plan_set_variant(mp._plan(a, be.fpdtype)[0], variant)
+    for kern in [one, *sep]:
+        kern.run(be.stream)
+    be.wait()
+    assert np.array_equal(c.get(), d.get())
+    ref = np.einsum('mk,ikn->imn', a._host,
+                    b.get().reshape(3, k, -1)).reshape(3*m, 5, neles)
+    assert rel_l2(c.get(), ref) < (1e-13 if precision == 'double' else 2e-6)
+    with pytest.raises(ValueError):
+        be.kernel('mul_slabs', a, b, c, 2)
+
+
+@pytest.mark.parametrize('precision', ['double', 'single'])
 @pytest.mark.parametrize('per_element', [True, False])
 @pytest.mark.parametrize('ep,last', [(1, 0), (2, 0), (2, 1)])
 def test_dense_epilogues(backend_factory, precision, per_element, ep, last):
