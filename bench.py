@@ -88,7 +88,7 @@ def make_mesh(c):
 #    written once, read-modify-write counted twice)
 def kernel_bytes(k, isz, nvars=5):
     name = k.name
-    if name == 'mul':
+    if name in ('mul', 'mul_slabs'):
         a, b, c = k.mats
         beta = k.rtargs.get('beta', 0.0)
         return (b.nrow + c.nrow*(1 + (beta != 0)))*b.ncol*isz + a.nrow*a.ncol*0
@@ -130,6 +130,26 @@ def kernel_bytes(k, isz, nvars=5):
         if ep == 3:
             by += 2*out.nrow*n*8                     # FP64 solution r/w
         return by
+    if name.startswith('hexdiv'):
+        # flux, divergence and correction (hexdivc: of a stored divergence)
+        u, fn, out, rcp, geo = k.mats
+        ep = int(name.rsplit('ep', 1)[1])
+        pts = out.nrow*out.ncol*isz
+        # u holds one row per point (hexdivc: of a wider bank); the next
+        # stage's traces go back to fn
+        by = 2*pts + fn.nrow*fn.ncol*(1 + k.disu)*isz
+        by += (rcp.nrow*rcp.ncol + (0 if geo is None else geo.nrow*geo.ncol))*isz
+        by += {2: 2*pts, 4: pts, 3: 2*pts//isz*8, 5: 2*pts//isz*8,
+               10: 2*pts, 11: 3*pts, 12: 3*pts, 13: 2*pts}.get(ep, 0)
+        return by
+    if name.startswith('hexns'):
+        u, comm, dv, grad, geo = k.mats
+        nf = grad.nrow//3       # dv takes one row per point; _nfv one side
+        rows = 2*u.nrow + nf*(2 if name.endswith('_nfv') else 4)
+        return (rows*u.ncol + geo.nrow*geo.ncol)*isz
+    if name == 'intcflux_nfv':
+        ul = k.views[0]
+        return ul.n*(4*nvars*isz + 2*nvars*isz + 3*isz + 4*4)
     if name.startswith('tdivf_flux_ep'):
         ep = int(name[-1])
         a0, a1, u, sm, fn, out, rcp = k.mats
@@ -154,7 +174,8 @@ def rhs_kernel_list(be, integ, c, precision):
     mixed = precision == 'mixed'
     if c['scheme'] == 'rk45' and sysm.fused_stages:
         # the graph of a middle RK45 stage (RHS fused with its update)
-        key = [k for k in sysm._kcache if len(k) == 5 and k[3] == 1][0]
+        key = [k for k in sysm._kcache
+               if len(k) == 7 and k[0] != 'rk4' and k[3] == 1][0]
         return flatten(sysm._kcache[key][0].klist)
     g = sysm._rhs_graphs(*((1, 1) if mixed else (0, 1)))[0]
     kerns = flatten(g.klist)
@@ -186,8 +207,8 @@ def measured_traffic(c, precision, label):
 def kernel_label(k):
     """Timing label: the kernel name plus the operator shape for operator
     applications (different element types stay apart)."""
-    if k.name == 'mul':
-        return f'mul{k.mats[0].nrow}x{k.mats[0].ncol}'
+    if k.name in ('mul', 'mul_slabs'):
+        return f'{k.name}{k.mats[0].nrow}x{k.mats[0].ncol}'
     if k.name.startswith('mul2_ep') or k.name.startswith('tdivf_flux'):
         a0, a1 = k.mats[:2]
         return f'{k.name}_{a0.nrow}x{a0.ncol}+{a1.ncol}'
@@ -199,9 +220,9 @@ def kernel_flops(k):
     column); 0 for everything else."""
     if getattr(k, 'kind', None) != 'dense':
         return 0
-    if k.name == 'mul':
+    if k.name in ('mul', 'mul_slabs'):
         a, b = k.mats[:2]
-        return 2*a.nrow*a.ncol*b.ncol
+        return 2*a.nrow*a.ncol*b.ncol*(b.nrow//a.ncol)
     a0, a1, b0 = k.mats[:3]
     return 2*a0.nrow*(a0.ncol + a1.ncol)*b0.ncol   # mul2 / tdivf_flux
 
