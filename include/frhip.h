@@ -110,12 +110,13 @@ int frhip_mul_slabs(void *plan, int n, int ncol, const void *b, long ldb,
 int frhip_mul(void *plan, int ncol, const void *b, long ldb, void *c,
               long ldc, double alpha, double beta, void *stream);
 
-/* Autotune a dense plan for (ncol, ldb): times the scalar kernel and the
- * MFMA kernel at 1, 2 and 4 wavefronts per block, each with the operator
- * read through the L2 or staged in LDS once per block, on the given input,
- * writing only to a scratch output, and keeps the fastest (*variant: 0
- * scalar, 1/2/4 wavefronts per block, +16 for the LDS-staged form; -1 for
- * structured plans, which have no variants).
+/* Autotune a dense plan for (ncol, ldb): times the MFMA kernel at 1, 2 and 4
+ * wavefronts per block, each with the operator read through the L2 or staged
+ * in LDS once per block, and with its rows split further while the grid is
+ * short of wavefronts, on the given input, writing only to a scratch output,
+ * and keeps the fastest (*variant: 0 scalar, 1/2/4 wavefronts per block, +16
+ * for the LDS-staged form, + 256 s in s row groups; -1 for structured plans,
+ * which have no variants).
  * Synchronous (uses the null stream); the input must be ready.  Replaces
  * the reference's rocBLAS solution-index sweep (pyfr/backends/hip/
  * rocblas.py:139-177). */
