@@ -144,12 +144,16 @@ def kernel_bytes(k, isz, nvars=5):
         return by
     if name.startswith('hexns'):
         u, comm, dv, grad, geo = k.mats
-        nf = grad.nrow//3       # dv takes one row per point; _nfv one side
-        rows = 2*u.nrow + nf*(2 if name.endswith('_nfv') else 4)
-        return (rows*u.ncol + geo.nrow*geo.ncol)*isz
+        # dv takes one row per point; _nfv writes one side's flux, without
+        # the density's
+        n, nf = u.ncol, grad.nrow//3
+        by = (2*u.nrow + nf)*n + geo.nrow*geo.ncol
+        by += nf*n*(nvars - 1)//nvars if name.endswith('_nfv') else 3*nf*n
+        return by*isz
     if name == 'intcflux_nfv':
         ul = k.views[0]
-        return ul.n*(4*nvars*isz + 2*nvars*isz + 3*isz + 4*4)
+        # no viscous flux of the density
+        return ul.n*(4*nvars*isz + 2*(nvars - 1)*isz + 3*isz + 2*4)
     if name.startswith('tdivf_flux_ep'):
         ep = int(name[-1])
         a0, a1, u, sm, fn, out, rcp = k.mats
