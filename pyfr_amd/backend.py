@@ -1165,11 +1165,14 @@ class PointwiseProvider:
         return None if b is None else (ct.c_double*2)(*b)
 
     @staticmethod
-    def _ns_consts(tplargs):
+    def _ns_consts(tplargs, required=False):
+        """The constants of the viscous kernels.  required: a run without
+        mu, Pr, ldg-beta or ldg-tau is refused (KeyError)."""
         c = tplargs['c']
+        get = (lambda k, default: c[k]) if required else c.get
         return (ct.c_double*8)(
-            c['gamma'], c.get('mu', 0.0), c.get('Pr', 1.0),
-            c.get('ldg-beta', 0.0), c.get('ldg-tau', 0.0),
+            c['gamma'], get('mu', 0.0), get('Pr', 1.0),
+            get('ldg-beta', 0.0), get('ldg-tau', 0.0),
             1.0 if tplargs.get('visc_corr') == 'sutherland' else 0.0,
             c.get('cpTref', 1.0), c.get('cpTs', 0.0))
 
@@ -1282,7 +1285,9 @@ class PointwiseProvider:
         if artvisc is not None:
             raise NotSuitableError('artificial viscosity is not supported')
         gs = View.stride_args(gradul, gradur)
-        consts = self._ns_consts(tplargs)
+        # the interfaces are where an option that was left out or misspelt
+        # shows: no other kernel needs all four
+        consts = self._ns_consts(tplargs, required=True)
         if nfv:
             # one map serves both arrays where they differ by an offset
             delta = set(np.unique(gradul.mapping_np - ul.mapping_np)) | \
