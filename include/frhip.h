@@ -187,7 +187,8 @@ int frhip_hex_plan_destroy(void *plan);
  * the volume part of the transformed divergence (frhip_hex_nsvol) and
  * tdivtconf + negdivconf are applied.  f (6 n^2, 5, neles): the common
  * normal fluxes.  ep (1-3, 10-17), c, rcp (a value per point), xa, dta, dtb
- * and last as for frhip_mul2.  disu (stages that form a next input): f
+ * and last as for frhip_mul2; every leading dimension covers whole blocks of
+ * 64 elements (ldr >= 64*ceil(neles/64), others times their variables).  disu (stages that form a next input): f
  * receives M0 of that input.  c and xa may be u.  base: as frhip_tflux_euler. */
 int frhip_hex_div(void *plan, int geo, int neles, const void *u, long ldu,
                   const void *gm, long ldg, void *f, long ldf, void *c,
@@ -199,7 +200,8 @@ int frhip_hex_div(void *plan, int geo, int neles, const void *u, long ldu,
  * baseadvecdiff/elements.py:47-55) + tdisf fused (pyfr/solvers/navstokes/
  * kernels/tflux.mako:13-50) + tdivtpcorf + gradcoru_fpts (baseadvecdiff/
  * elements.py:87-101).  u (n^3, 5, neles), cm (6 n^2, 5, neles) the common
- * solution; gm, rcp the metric terms (rcp: geo = FRHIP_GEO_CURVED); dv
+ * solution; gm, rcp the metric terms (rcp: geo = FRHIP_GEO_CURVED, its rows
+ * whole blocks of 64 elements); dv
  * (n^3, 5, neles) receives the volume part of the transformed divergence
  * and g the physical gradients at the flux points (3, 6 n^2, 5, neles),
  * which may hold cm in its first 6 n^2 rows, or, with nfv (linear hexes),

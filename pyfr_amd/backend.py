@@ -907,7 +907,8 @@ class HexLineProvider:
         nu, nf = basis.nupts, basis.nfpts
         if (u.nrow < nu or fn.nrow != nf or out.nrow != nu or
                 any(m.ncol != out.ncol or m.dtype != out.dtype
-                    for m in (u, fn)) or rcpdjac.nrow != nu):
+                    for m in (u, fn)) or rcpdjac.nrow != nu or
+                5*rcpdjac.leaddim < out.ncol):
             raise ValueError('Incompatible matrices for hexdiv')
         plan = self._plan(basis, out.dtype)
         if ep in (3, 14, 15, 16, 17) and out.dtype != np.float32:
@@ -947,7 +948,8 @@ class HexLineProvider:
         if (u.nrow != nu or comm.nrow < nf or dv.nrow < nu or
                 grad.nrow != 3*nf or any(m.ncol != u.ncol or
                                          m.dtype != u.dtype
-                                         for m in (comm, dv, grad))):
+                                         for m in (comm, dv, grad)) or
+                (geo == 0 and 5*rcpdjac.leaddim < u.ncol)):
             raise ValueError('Incompatible matrices for hexns')
         plan = self._plan(basis, u.dtype)
         base = PointwiseProvider._base(tplargs)

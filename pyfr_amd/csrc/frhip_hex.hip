@@ -1024,13 +1024,14 @@ int frhip_hex_div(void *plan, int geo, int neles, const void *u, long ldu,
              "the precision form's epilogues need FP32 operands");
     FR_CHECK(ep < 2 || xa, "RK epilogue needs the r1 / accumulator array");
     FR_CHECK(neles >= 0, "invalid extents");
+    // the last block's lanes past neles read (and drop) whole blocks of 64
     const long ncol = 320L*((neles + 63L)/64);
     FR_CHECK(ldu >= ncol && ldf >= ncol && ldc >= ncol &&
-             (geo < 0 || ldg*5 >= ncol*3) && ldr >= neles,
+             (geo < 0 || ldg*5 >= ncol*3) && ldr*5 >= ncol,
              "invalid leading dimensions");
     // lane offsets are 32-bit byte offsets of up to n^2 rows
     const size_t esz = p->dtype == FRHIP_F64 ? 8 : 4;
-    const long ldmax = std::max(std::max(ldu, ldf), std::max(ldc, ldg));
+    const long ldmax = std::max({ldu, ldf, ldc, ldg, ldr});
     FR_CHECK((size_t)(p->n*p->n*ldmax)*(ep == 3 || ep >= 14 ? 8 : esz) <
                  (size_t)1 << 32, "leading dimension too large");
     FR_CHECK(!disu || (ep >= 2 && !(last && ep <= 3)),
@@ -1061,7 +1062,8 @@ int frhip_hex_nsvol(void *plan, int geo, int neles, const void *u, long ldu,
     FR_CHECK(neles >= 0, "invalid extents");
     const long ncol = 320L*((neles + 63L)/64);
     FR_CHECK(ldu >= ncol && ldcm >= ncol && ldd >= ncol && ldgr >= ncol &&
-             ldg*5 >= ncol*3, "invalid leading dimensions");
+             ldg*5 >= ncol*3 && (geo != FRHIP_GEO_CURVED || ldr*5 >= ncol),
+             "invalid leading dimensions");
     // the vertices of a lane are addressed by 32-bit byte offsets
     FR_CHECK((size_t)(neles + 63)*24 < (size_t)1 << 32, "too many elements");
     if (neles == 0) return 0;

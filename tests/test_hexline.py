@@ -184,3 +184,81 @@ class _Faces:
         e = FluidElements(HexShape, mesh.spts['hex'], cfg)
         self.nfacefpts = e.nfacefpts
         self.get_pnorms_for_inters = e.get_pnorms_for_inters
+
+
+def _hex_args(be, order, neles):
+    """Operands of the two entry points for neles elements, every one of
+    them padded to a whole block of 64."""
+    sh = HexShape(order)
+    rng = np.random.default_rng(1)
+    m = {k: be.matrix((r, 5, neles), 1 + rng.random((r, 5, neles)),
+                      tags={'align'})
+         for k, r in (('u', sh.nupts), ('f', sh.nfpts), ('c', sh.nupts),
+                      ('g', 3*sh.nfpts))}
+    m['s'] = be.matrix((3, sh.nupts, 3, neles),
+                       rng.random((3, sh.nupts, 3, neles)), tags={'align'})
+    m['r'] = be.matrix((sh.nupts, neles), 1 + rng.random((sh.nupts, neles)),
+                       tags={'align'})
+    return sh, m
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('precision', ['double', 'single'])
+@pytest.mark.parametrize('order,neles', [(2, 1), (2, 65), (4, 100)])
+def test_short_metric_rows_are_refused(backend_factory, precision, order,
+                                       neles):
+    """1/|J| rows that do not cover the last block, which every lane of it
+    reads.  (The arrays themselves do: nothing here reads past them.)"""
+    import ctypes as ct
+    from pyfr_amd._lib import FrHipError
+    from pyfr_amd.backend import HexLineProvider
+    be = backend_factory(precision=precision)
+    sh, m = _hex_args(be, order, neles)
+    hp = next(p for p in be._providers if isinstance(p, HexLineProvider))
+    plan = hp._plan(sh, be.fpdtype)
+    u, f, c, g, s, r = (m[k] for k in 'ufcgsr')
+    consts = (ct.c_double*8)(1.4, 1e-3, 0.7, 0, 0, 0, 1, 0)
+
+    def div(ldr):
+        be.lib.hex_div(plan, 0, neles, u.data, u.leaddim, s.data, s.leaddim,
+                       f.data, f.leaddim, c.data, c.leaddim, 1, r.data, ldr,
+                       None, 0.0, 0.0, 0, 0, 1.4, None, be.stream)
+
+    def ns(ldr):
+        be.lib.hex_nsvol(plan, 0, neles, u.data, u.leaddim, f.data,
+                         f.leaddim, s.data, s.leaddim, r.data, ldr, c.data,
+                         c.leaddim, g.data, g.leaddim, 0, consts, None,
+                         be.stream)
+    print(f'\n[hexline ldr] {precision} p={order} {neles}', flush=True)
+    for call in (div, ns):
+        for ldr in (neles, r.leaddim - 1):
+            with pytest.raises(FrHipError, match='leading dimensions'):
+                call(ldr)
+        call(r.leaddim)
+    be.wait()
+    assert np.isfinite(c.get()).all() and np.isfinite(g.get()).all()
+
+
+@pytest.mark.parametrize('order,neles', [(2, 1), (4, 100)])
+def test_unaligned_metric_is_refused(monkeypatch, order, neles):
+    """The same at the kernel providers, on the host."""
+    import pyfr_amd._lib as _lib
+    from pyfr_amd.backend import AMDBackend
+    from tests.test_ns_options import StubLib
+    monkeypatch.setattr(_lib, '_lib', StubLib())
+    be = AMDBackend(make_cfg('navier-stokes', order))
+    sh, m = _hex_args(be, order, neles)
+    short = be.matrix((sh.nupts, neles))
+    tpl = {'c': {'gamma': 1.4}}
+
+    def div(r):
+        be.kernel('hexdiv', sh, 0, neles, m['u'], m['f'], m['c'], r, 1.4,
+                  m['s'])
+
+    def ns(r):
+        be.kernel('hexns', sh, 0, neles, m['u'], m['f'], m['c'], m['g'], tpl,
+                  m['s'], r)
+    for make in (div, ns):
+        make(m['r'])
+        with pytest.raises(ValueError, match='Incompatible'):
+            make(short)
