@@ -143,11 +143,12 @@ def kernel_bytes(k, isz, nvars=5):
                10: 2*pts, 11: 3*pts, 12: 3*pts, 13: 2*pts}.get(ep, 0)
         return by
     if name.startswith('hexns'):
-        u, comm, dv, grad, geo = k.mats
+        u, comm, dv, grad, geo, fnorms = k.mats
         # dv takes one row per point; _nfv writes one side's flux, without
         # the density's
         n, nf = u.ncol, grad.nrow//3
         by = (2*u.nrow + nf)*n + geo.nrow*geo.ncol
+        by += 0 if fnorms is None else fnorms.nrow*fnorms.ncol
         by += nf*n*(nvars - 1)//nvars if name.endswith('_nfv') else 3*nf*n
         return by*isz
     if name == 'intcflux_nfv':

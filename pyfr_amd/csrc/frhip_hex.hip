@@ -519,6 +519,7 @@ struct HexNsArgs {
     long ldg;
     const T *rcp;
     long ldr;
+    const T *fn;        // NFV: the faces' normals, rows of ldg
     T *dv;              // volume part of the transformed divergence
     long ldd;
     T *g;               // gradients (3, nfpts, 5, E) or normal viscous flux
@@ -605,7 +606,10 @@ struct HexFace {
 // LDS buffer; all of the (3, Nu, 5) and (3, Nf, 5) intermediates of the
 // kernels replaced stay in registers and LDS.  NFV: at the flux points only
 // the normal viscous flux of this side (4 values) instead of the gradients
-// (15), for meshes whose interface kernel needs no more.
+// (15), for meshes whose interface kernel needs no more.  The normal comes
+// from coefficients formed in FP64 and rounded once: rebuilt from FP32
+// vertices it was off by 4e-6 of its length on 48^3 elements of [0, 2 pi],
+// 8e-5 with the box at 100.
 template <typename T, int N, int GEO, bool NFV, int EB>
 __global__ __launch_bounds__(N*N*N*EB)
 __attribute__((amdgpu_waves_per_eu(4))) void k_hex_nsvol(
@@ -729,31 +733,16 @@ __attribute__((amdgpu_waves_per_eu(4))) void k_hex_nsvol(
         const HexFace h = HexFace::of<N>(q);
         int p0, st;
         h.line<N>(p0, st);
-        // this side's normal from the tangents along the face's axes (its
-        // four vertices), and its state
+        // this side's normal (linear in each of the face's coordinates: their
+        // product's coefficient vanishes) and its state
         T nf[3] = {}, uf[5] = {};
         if constexpr (NFV) {
-            T ts[3], tt[3];
-            const int sa = h.axis == 0 ? 1 : 0, ta = h.axis == 2 ? 1 : 2;
-            const int v0 = h.side << h.axis;
             const T x = line->x[h.a], y = line->x[h.b];
-            const T *gv = a.geo + soa_ix(e, 0, 3);
+            const T *gn = a.fn + 3*(q/NN)*a.ldg + soa_ix(e, 0, 3);
 #pragma unroll
-            for (int b = 0; b < 3; ++b) {
-                const T w00 = gv[v0*a.ldg + b*SOA];
-                const T w10 = gv[(v0 | 1 << sa)*a.ldg + b*SOA];
-                const T w01 = gv[(v0 | 1 << ta)*a.ldg + b*SOA];
-                const T w11 = gv[(v0 | 1 << sa | 1 << ta)*a.ldg + b*SOA];
-                ts[b] = T(0.25)*((T(1) - y)*(w10 - w00) +
-                                 (T(1) + y)*(w11 - w01));
-                tt[b] = T(0.25)*((T(1) - x)*(w01 - w00) +
-                                 (T(1) + x)*(w11 - w10));
-            }
-            PencilGeo<T>::cross(ts, tt, nf);
-            // axes (y, z), (x, z), (x, y): the middle pair is left-handed
-            const T sg = (h.axis == 1) != (h.side == 0) ? T(-1) : T(1);
-#pragma unroll
-            for (int b = 0; b < 3; ++b) nf[b] *= sg;
+            for (int b = 0; b < 3; ++b)
+                nf[b] = fma(y, gn[2*a.ldg + b*SOA],
+                            fma(x, gn[a.ldg + b*SOA], gn[b*SOA]));
             layer_end(nf);
 #pragma unroll
             for (int m = 0; m < N; ++m) {
@@ -926,13 +915,13 @@ constexpr int hex_ns_eb()
 }
 
 template <typename T, int N>
-static int hex_ns_n(const HexPlan *p, int geo, int nfv, const HexNsArgs<T> &a,
+static int hex_ns_n(const HexPlan *p, int geo, const HexNsArgs<T> &a,
                     hipStream_t s)
 {
     constexpr int EB = hex_ns_eb<T, N>();
     const dim3 grid(cdiv(a.neles, EB)), block(N*N*N*EB);
     const auto *line = static_cast<const HexLine<T, N> *>(p->line);
-    auto k = nfv ? k_hex_nsvol<T, N, FRHIP_GEO_HEX_LINEAR, true, EB>
+    auto k = a.fn ? k_hex_nsvol<T, N, FRHIP_GEO_HEX_LINEAR, true, EB>
            : geo == FRHIP_GEO_HEX_LINEAR
                ? k_hex_nsvol<T, N, FRHIP_GEO_HEX_LINEAR, false, EB>
                : k_hex_nsvol<T, N, FRHIP_GEO_CURVED, false, EB>;
@@ -942,22 +931,23 @@ static int hex_ns_n(const HexPlan *p, int geo, int nfv, const HexNsArgs<T> &a,
 }
 
 template <typename T>
-static int hex_ns_t(const HexPlan *p, int geo, int nfv, int neles,
+static int hex_ns_t(const HexPlan *p, int geo, const void *fn, int neles,
                     const void *u, long ldu, const void *cm, long ldcm,
                     const void *gm, long ldg, const void *rcp, long ldr,
                     void *dv, long ldd, void *g, long ldgr,
                     const double *consts, const double *base, hipStream_t s)
 {
     const HexNsArgs<T> a{neles, (const T *)u, ldu, (const T *)cm, ldcm,
-                         (const T *)gm, ldg, (const T *)rcp, ldr, (T *)dv,
-                         ldd, (T *)g, ldgr, ns_consts<T>(consts, -1.0),
+                         (const T *)gm, ldg, (const T *)rcp, ldr,
+                         (const T *)fn, (T *)dv, ldd, (T *)g, ldgr,
+                         ns_consts<T>(consts, -1.0),
                          base ? base_state<T>(base, consts[0])
                               : BaseState<T>{}};
     switch (p->n) {
-        case 2: return hex_ns_n<T, 2>(p, geo, nfv, a, s);
-        case 3: return hex_ns_n<T, 3>(p, geo, nfv, a, s);
-        case 4: return hex_ns_n<T, 4>(p, geo, nfv, a, s);
-        default: return hex_ns_n<T, 5>(p, geo, nfv, a, s);
+        case 2: return hex_ns_n<T, 2>(p, geo, a, s);
+        case 3: return hex_ns_n<T, 3>(p, geo, a, s);
+        case 4: return hex_ns_n<T, 4>(p, geo, a, s);
+        default: return hex_ns_n<T, 5>(p, geo, a, s);
     }
 }
 
@@ -1050,14 +1040,14 @@ int frhip_hex_div(void *plan, int geo, int neles, const void *u, long ldu,
 int frhip_hex_nsvol(void *plan, int geo, int neles, const void *u, long ldu,
                     const void *cm, long ldcm, const void *gm, long ldg,
                     const void *rcp, long ldr, void *dv, long ldd, void *g,
-                    long ldgr, int nfv, const double *consts,
+                    long ldgr, const void *fn, const double *consts,
                     const double *base, void *stream)
 {
     FR_API_BEGIN
     HexPlan *p = static_cast<HexPlan *>(plan);
     FR_CHECK(p && u && cm && gm && dv && g && consts, "null argument");
     FR_CHECK(geo == FRHIP_GEO_HEX_LINEAR ||
-             (geo == FRHIP_GEO_CURVED && rcp && !nfv),
+             (geo == FRHIP_GEO_CURVED && rcp && !fn),
              "invalid geometry mode");
     FR_CHECK(neles >= 0, "invalid extents");
     const long ncol = 320L*((neles + 63L)/64);
@@ -1069,9 +1059,9 @@ int frhip_hex_nsvol(void *plan, int geo, int neles, const void *u, long ldu,
     if (neles == 0) return 0;
     hipStream_t s = as_stream(stream);
     return p->dtype == FRHIP_F64
-        ? hex_ns_t<double>(p, geo, nfv, neles, u, ldu, cm, ldcm, gm, ldg, rcp,
+        ? hex_ns_t<double>(p, geo, fn, neles, u, ldu, cm, ldcm, gm, ldg, rcp,
                            ldr, dv, ldd, g, ldgr, consts, base, s)
-        : hex_ns_t<float>(p, geo, nfv, neles, u, ldu, cm, ldcm, gm, ldg, rcp,
+        : hex_ns_t<float>(p, geo, fn, neles, u, ldu, cm, ldcm, gm, ldg, rcp,
                           ldr, dv, ldd, g, ldgr, consts, base, s);
     FR_API_END
 }

@@ -16,6 +16,8 @@ evaluated directly rather than through an orthonormal Vandermonde inverse.
 """
 import numpy as np
 
+from pyfr_amd.shapes import HEX_FACES
+
 
 def _lagrange_1d(x, pts):
     """Values and derivatives of the Lagrange basis through x at pts."""
@@ -83,6 +85,28 @@ def hex_corner_index(k):
     n = k + 1
     return [((v & 1)*k) + n*((((v >> 1) & 1)*k) + n*(((v >> 2) & 1)*k))
             for v in range(8)]
+
+
+def linear_hex_face_normals(v):
+    """Unnormalised outward normals of trilinear hexes with vertices v (8,
+    neles, 3), as coefficients (18, 3, neles): on face f, at its coordinates
+    (x, y), row 3f + x row 3f + 1 + y row 3f + 2.  The tangents are a + y c
+    and b + x c, so x y has none."""
+    out = np.empty((18, 3, v.shape[1]))
+    for f, (nax, side, sax, tax) in enumerate(HEX_FACES):
+        # vertex w: bit d set on the high side of axis d
+        o = (side > 0) << nax
+        w00, w10, w01, w11 = (v[o | i << sax | j << tax]
+                              for j in (0, 1) for i in (0, 1))
+        a = 0.25*((w10 - w00) + (w11 - w01))
+        b = 0.25*((w01 - w00) + (w11 - w10))
+        c = 0.25*((w11 - w01) - (w10 - w00))
+        # (s, t, normal axis) is right-handed but for the y faces
+        sg = side if nax != 1 else -side
+        for i, n in enumerate((np.cross(a, b), np.cross(a, c),
+                               np.cross(c, b))):
+            out[3*f + i] = sg*n.T
+    return out
 
 
 def shape_basis():

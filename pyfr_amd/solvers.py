@@ -36,7 +36,8 @@ import time
 import numpy as np
 
 from pyfr_amd.geometry import (AffineGeometry, CurvedSimplexGeometry,
-                               HexGeometry, hex_corner_index)
+                               HexGeometry, hex_corner_index,
+                               linear_hex_face_normals)
 from pyfr_amd.mesh import sorted_face_fpts, sorted_face_fpts_structured
 from pyfr_amd.shapes import SHAPES as HEX_SHAPES
 from pyfr_amd.simplex import SIMPLEX_SHAPES
@@ -413,6 +414,13 @@ class FluidElements:
             v.transpose(0, 2, 1)), tags={'align'})
 
     @cached_property
+    def _fnorms_linear(self):
+        # rows of the vertices' length: (18, ndims, neles)
+        v = self.eles[hex_corner_index(self.geom.sorder), self.linoff:]
+        return self._be.const_matrix(linear_hex_face_normals(v),
+                                     tags={'align'})
+
+    @cached_property
     def _upts_const(self):
         return self._be.const_matrix(self.basis.upts)
 
@@ -757,7 +765,8 @@ class NavierStokesElements(EulerElements):
                     'hexns', self.basis, mode, n, s(self.scal_upts[uin]),
                     s(self._vect_fpts), s(self._vect_upts),
                     s(self._vect_fpts), tplargs | self.base_tpl, metric,
-                    s(self._rcpdjac_upts), nfv=nfv))
+                    s(self._rcpdjac_upts),
+                    fnorms=self._fnorms_linear if nfv else None))
 
             def hexdiv(fout, xa=None, stage=None, disu=False):
                 return be.kernel(

@@ -157,6 +157,43 @@ def test_ns_steps(backend_factory, scheme, precision, n, order):
     assert rel_l2(got, ref) < tol
 
 
+def _offset(x, y, z):
+    return x + 100.0 + 0.05*np.sin(y), y - 100.0 + 0.03*np.sin(z), z + 50.0
+
+
+@pytest.mark.parametrize('order', [2, 4])
+def test_face_normals(monkeypatch, order):
+    """The normals that the viscous flux at the interfaces is taken along:
+    those of the stored metric, and in single precision one rounding of
+    each coefficient from it, wherever the mesh lies."""
+    import pyfr_amd._lib as _lib
+    from pyfr_amd.backend import AMDBackend
+    from tests.test_ns_options import StubLib
+    monkeypatch.setattr(_lib, '_lib', StubLib())
+    # 1.2e-7: half an ulp of each of three coefficients, the largest of them
+    # the normal itself.  The stored metric's own rounding: it is a
+    # derivative of X x X_a, which is a derivative too, in components of two
+    # products of up to 106.3 and 1.05 (half an edge), on normals of 0.3 and
+    # more; the derivative matrices' rows sum to at most 2 p^2 in modulus
+    meps = 2.2e-16*2*106.3*1.05/0.3*(2*order*order)**2
+    for precision, eps in (('double', meps), ('single', 1.2e-7)):
+        cfg = make_cfg('navier-stokes', order, precision=precision)
+        integ = get_integrator(AMDBackend(cfg),
+                               BoxMesh((5, 4, 3), warp=_offset), cfg)
+        e = integ.system.ele_map['hex']
+        assert e.linoff == 0
+        # (18, ndims, neles), as the kernel reads them
+        c = e._fnorms_linear._host.astype(e._fnorms_linear.dtype)
+        c = c.astype(float).reshape(6, 3, 3, e.neles)
+        x = HexShape(order).x1d
+        xy = np.array([(1, a, b) for b in x for a in x])
+        got = np.einsum('pi,fice->fpec', xy, c)
+        ref = e._pnorm_fpts.reshape(got.shape)
+        mag = np.sqrt((ref**2).sum(axis=-1))
+        assert mag.min() > 0.3
+        assert (np.abs(got - ref).max(axis=-1)/mag).max() < eps
+
+
 def test_normals_match_is_checked():
     """A periodic pair of faces whose vertices differ beyond rounding keeps
     the gradients at its interfaces."""
