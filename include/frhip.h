@@ -232,9 +232,10 @@ int frhip_hex_nsvol(void *plan, int geo, int neles, const void *u, long ldu,
  * variant 64: the 4x4x1 MFMA form, 65: the same in blocks of the five
  * wavefronts of an element block (one workgroup, so one XCD's L2 serves
  * every variable's reads of u), 66: with the operator staged in LDS, each
- * of the three + 256 s: its rows split over s row groups.  The variants are
- * timed with an RK4 stage's epilogue.  c may be u itself (an RHS in place):
- * such a call runs variant 32, whose block barriers order every read of u
+ * of the three + 256 s: its rows split over s row groups.  plan_tune times
+ * the plain store, plan_tune_rk4 the stages' epilogues for ep 10..13 (which
+ * otherwise run the former's choice); set_variant sets both.  c may be u
+ * itself (an RHS in place): such a call runs variant 32, whose block barriers order every read of u
  * before any write of c, whatever the plan's variant.
  * ep 10..13: RK4 stages 1..4 on four registers, with the update axnpby of
  * pyfr/integrators/explicit/steppers.py:67-108 in the epilogue (k = the
@@ -251,6 +252,9 @@ int frhip_tdivf_plan_destroy(void *plan);
 int frhip_tdivf_plan_tune(void *plan, int ncol, const void *u, long ldu,
                           const void *smats, long lds, const void *fn,
                           long ldf, double gamma, int reps, int *variant);
+int frhip_tdivf_plan_tune_rk4(void *plan, int ncol, const void *u, long ldu,
+                              const void *smats, long lds, const void *fn,
+                              long ldf, double gamma, int reps, int *variant);
 int frhip_tdivf_plan_set_variant(void *plan, int variant);
 int frhip_tdivf_flux_euler(void *plan, int ncol, const void *u, long ldu,
                            const void *smats, long lds, const void *fn,

@@ -70,6 +70,8 @@ _FUNCS = {
     'frhip_tdivf_plan_destroy': [_P],
     'frhip_tdivf_plan_tune': [_P, _I, _P, _L, _P, _L, _P, _L, _D, _I,
                               ct.POINTER(_I)],
+    'frhip_tdivf_plan_tune_rk4': [_P, _I, _P, _L, _P, _L, _P, _L, _D,
+                                  _I, ct.POINTER(_I)],
     'frhip_tdivf_plan_set_variant': [_P, _I],
     'frhip_tdivf_flux_euler': [_P, _I, _P, _L, _P, _L, _P, _L, _P, _L, _I,
                                _P, _L, _P, _D, _D, _I, _D, _P],

@@ -782,9 +782,9 @@ class MulProvider:
                            xa)
 
     def tuning_report(self):
-        """The variant the tuner chose for each dense plan and shape
-        (0: scalar kernel; 1, 2, 4: matrix-core kernel, wavefronts per
-        block)."""
+        """The variant the tuner chose for each dense plan and shape (1, 2,
+        4: matrix-core kernel, wavefronts per block; others as in
+        include/frhip.h); tdivf_flux_rk4: for RK4 stages."""
         shapes = {}
         for plan, _, a in self._plans.values():
             shapes[plan] = ('mul', f'{a.nrow}x{a.ncol}')
@@ -795,6 +795,8 @@ class MulProvider:
         out = []
         for key, v in self._tuned.items():
             kind, shape = shapes.get(key[0], ('?', '?'))
+            if kind == 'tdivf_flux' and key[2]:
+                kind += '_rk4'
             out.append({'kernel': kind, 'operator': shape, 'ncol': key[1],
                         'variant': v})
         return out
@@ -831,13 +833,15 @@ class MulProvider:
             self._plans3[key] = (plan.value, a0, a1)
         plan = self._plans3[key][0]
         ncol = out.ncol
-        if self.backend.autotune and (plan, ncol) not in self._tuned:
+        # right-hand sides and RK4 stages each keep a variant of their own
+        rk4 = ep >= 10
+        if self.backend.autotune and (plan, ncol, rk4) not in self._tuned:
             self.backend.wait()
             v = ct.c_int()
-            lib.tdivf_plan_tune(plan, ncol, u.data, u.leaddim, smats.data,
-                                smats.leaddim, fn.data, fn.leaddim, gamma, 5,
-                                ct.byref(v))
-            self._tuned[(plan, ncol)] = v.value
+            tune = lib.tdivf_plan_tune_rk4 if rk4 else lib.tdivf_plan_tune
+            tune(plan, ncol, u.data, u.leaddim, smats.data, smats.leaddim,
+                 fn.data, fn.leaddim, gamma, 5, ct.byref(v))
+            self._tuned[(plan, ncol, rk4)] = v.value
         _check_xa(xa, out, ep)
         if ep >= 10:
             # RK4 stages: xa = (r1, r0) with the step's device scalar

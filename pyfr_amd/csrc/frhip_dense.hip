@@ -1429,7 +1429,9 @@ int bf16_launch(const Bf16Plan *p, int ep, long ncol, const void *b0,
 // ---- flux-fused plans -----------------------------------------------------
 
 struct FluxPlan {
-    DensePlan d;        // m, k0 = 3 nupts, k1 = nfpts, fragments
+    DensePlan d;        // m, k0 = 3 nupts, k1 = nfpts, fragments; variant
+                        // of all epilogues but
+    int vrk4;           // those of RK4 stages (-1: not chosen, as the others)
     int nupts, nq;
     void *af4;          // FP32: k_tdivf_flux4 fragments, or null
     int g4, nc0, nc1;   // 4-row groups, flux and fn chunks
@@ -1607,7 +1609,8 @@ static int flux_launch(const FluxPlan *p, int ep, long ncol, const void *u,
     FR_CHECK(ep == 0 || rcp, "epilogue needs 1/|J|");
     FR_CHECK(ep < 2 || xa, "RK epilogue needs the r1 / accumulator array");
     const size_t esz = p->d.dtype == FRHIP_F64 ? 8 : 4;
-    int wpb = p->d.variant > 0 ? p->d.variant : 4;
+    int wpb = ep >= 10 && p->vrk4 > 0 ? p->vrk4
+            : p->d.variant > 0 ? p->d.variant : 4;
     if (is_flux4(wpb) && (!p->af4 ||
                           !flux4_valid(wpb, p->g4, p->nc0 + p->nc1)))
         wpb = 4;
@@ -1628,6 +1631,116 @@ static int flux_launch(const FluxPlan *p, int ep, long ncol, const void *u,
                                ldc, rcp, ldr, xa, dta, dtb, gamma, s);
     if (rc) return rc;
     FR_LAUNCHED();
+    return 0;
+}
+
+// Times the variants and keeps the fastest in `chosen`: those of plain
+// right-hand sides with the plain store, those of RK4 steps with the four
+// stages' epilogues in turn, on scratch registers.  One choice does not
+// serve both: p = 4 prisms, 9,216 of them, took 63 us in the 16-row tiles
+// with the store and 150 with an epilogue; with the choice made for RK4,
+// right-hand sides of 16,000 p = 2 prisms took 41.0 us where the store's own
+// takes 38.9.  Nor does one stage speak for four: in the second one, 63,888
+// p = 2 tets take the block-cooperative form and the 4x4x1 form 20 us each,
+// in the last one 16.4 and 18.0.  (RK45 and Euler stages update the
+// register they read, which the block-cooperative form serves alone.)  The
+// least of three interleaved rounds counts: candidates lie within a few per
+// cent of each other.
+static int flux_tune(const FluxPlan *p, bool rk4, int &chosen, int ncol,
+                     const void *u, long ldu, const void *smats, long lds,
+                     const void *fn, long ldf, double gamma, int reps,
+                     int *variant)
+{
+    if (ncol == 0) {
+        if (variant) *variant = chosen;
+        return 0;
+    }
+    const size_t esz = p->d.dtype == FRHIP_F64 ? 8 : 4;
+    const size_t nb = ((size_t)p->d.m*ncol*esz + 255)/256*256;
+    char *scratch = nullptr;
+    if (rk4 && hipMalloc(&scratch, 3*nb + (size_t)ncol*esz + 256) !=
+                   hipSuccess) {
+        // a mesh that leaves no room for two more registers is timed with
+        // the store, which needs one
+        (void)hipGetLastError();
+        scratch = nullptr;
+        rk4 = false;
+    }
+    if (!rk4) FR_HIP(hipMalloc(&scratch, nb));
+    void *rcp = nullptr;
+    char *xa = nullptr;
+    if (rk4) {
+        rcp = scratch + 3*nb + 256;
+        xa = scratch + 3*nb;
+        void *const ptrs[4] = {scratch + nb, scratch + 2*nb, xa + 24,
+                               nullptr};
+        if (hipMemset(scratch, 0, 3*nb + (size_t)ncol*esz + 256) !=
+                hipSuccess ||
+            hipMemcpy(xa, ptrs, sizeof(ptrs), hipMemcpyHostToDevice) !=
+                hipSuccess) {
+            (void)hipFree(scratch);
+            set_error("tuning scratch");
+            return 1;
+        }
+    }
+    const size_t ldsb = (size_t)p->d.mt*(p->d.ks0 + p->d.ks1)*64*esz;
+    std::vector<int> cands = {1, 2, 4, FR_LDSV + 1, FR_LDSV + 2, FR_LDSV + 4,
+                              FR_BLKV, FR_V4, FR_V4B, FR_V4L};
+    // A split repeats the flux in every row group: only while the grid is
+    // short of four wavefronts per SIMD (p = 4 pyramids, 34,944 of them: 80
+    // us in two row groups, 98 in one; 196,608: 390 and 359).
+    int last = p->g4;
+    for (int s = 2; s <= p->g4; ++s) {
+        const int gw = flux4_group(p->g4, s*FR_SPLIT + FR_V4L);
+        if (gw == last) continue;
+        if (ncol/64*cdiv(p->g4, last) >= 4096) break;
+        last = gw;
+        cands.push_back(s*FR_SPLIT + FR_V4);
+        cands.push_back(s*FR_SPLIT + FR_V4L);
+    }
+    // the staged form of the smallest split whose operator fits in LDS
+    for (int s = 2; s <= p->g4; ++s)
+        if (flux4_valid(s*FR_SPLIT + FR_V4L, p->g4, p->nc0 + p->nc1)) {
+            cands.push_back(s*FR_SPLIT + FR_V4L);
+            break;
+        }
+    hipEvent_t e0, e1;
+    (void)hipEventCreate(&e0);
+    (void)hipEventCreate(&e1);
+    const int n = rk4 ? (reps + 3)/4*4 : reps;
+    float best = 1e30f;
+    int bestv = 4, rc = 0;
+    for (int round = 0; round < 3 && !rc; ++round)
+        for (int v : cands) {
+            if (is_flux4(v)
+                    ? !p->af4 || !flux4_valid(v, p->g4, p->nc0 + p->nc1)
+                    : v != FR_BLKV && !variant_valid(v, ldsb, false))
+                continue;
+            FluxPlan q = *p;
+            q.d.variant = q.vrk4 = v;
+            // the first launch is not timed
+            for (int it = 0; it < n + 1 && !rc; ++it) {
+                if (it == 1) (void)hipEventRecord(e0, nullptr);
+                rc = flux_launch(&q, rk4 ? 10 + it % 4 : 0, ncol, u, ldu,
+                                 smats, lds, fn, ldf, scratch, ncol, rcp, 0,
+                                 xa, 0, 0, gamma, nullptr);
+            }
+            if (rc) break;
+            (void)hipEventRecord(e1, nullptr);
+            (void)hipEventSynchronize(e1);
+            float ms = 0;
+            (void)hipEventElapsedTime(&ms, e0, e1);
+            if (ms < best) {
+                best = ms;
+                bestv = v;
+            }
+        }
+    (void)hipEventDestroy(e0);
+    (void)hipEventDestroy(e1);
+    (void)hipFree(scratch);
+    if (rc) return rc;
+    chosen = bestv;
+    if (variant) *variant = bestv;
     return 0;
 }
 
@@ -1716,7 +1829,7 @@ int frhip_tdivf_plan_create(void **plan, int m, int nupts, int nfpts,
         }
     }
     FluxPlan *p = new FluxPlan{{m, k0, nfpts, dtype, mt, ks0, ks1, d, nullptr,
-                                4}, nupts, nq, d4, g4, nc0, nc1};
+                                4}, -1, nupts, nq, d4, g4, nc0, nc1};
     *plan = p;
     return 0;
     FR_API_END
@@ -1763,83 +1876,20 @@ int frhip_tdivf_plan_tune(void *plan, int ncol, const void *u, long ldu,
     FR_API_BEGIN
     FluxPlan *p = static_cast<FluxPlan *>(plan);
     FR_CHECK(p && reps > 0, "invalid arguments");
-    const size_t esz = p->d.dtype == FRHIP_F64 ? 8 : 4;
-    // Timed with an RK4 stage's epilogue (10 + 1: both registers read and
-    // written) on scratch registers, as time steps run the kernel: the plain
-    // store ranks the variants differently (p = 4 prisms, 9,216 of them: 63
-    // us for the 16-row tiles with it, 150 with the epilogue).
-    if (ncol == 0) {
-        if (variant) *variant = p->d.variant;
-        return 0;
-    }
-    const size_t nb = ((size_t)p->d.m*ncol*esz + 255)/256*256;
-    char *scratch = nullptr;
-    FR_HIP(hipMalloc(&scratch, 3*nb + (size_t)ncol*esz + 256));
-    void *c = scratch, *rcp = scratch + 3*nb + 256;
-    char *xa = scratch + 3*nb;
-    void *const ptrs[4] = {scratch + nb, scratch + 2*nb, xa + 24, nullptr};
-    if (hipMemset(scratch, 0, 3*nb + (size_t)ncol*esz + 256) != hipSuccess ||
-        hipMemcpy(xa, ptrs, sizeof(ptrs), hipMemcpyHostToDevice) !=
-            hipSuccess) {
-        (void)hipFree(scratch);
-        set_error("tuning scratch");
-        return 1;
-    }
-    hipEvent_t e0, e1;
-    (void)hipEventCreate(&e0);
-    (void)hipEventCreate(&e1);
-    float best = 1e30f;
-    int bestv = 4, rc = 0;
-    const size_t ldsb = (size_t)p->d.mt*(p->d.ks0 + p->d.ks1)*64*esz;
-    std::vector<int> cands = {1, 2, 4, FR_LDSV + 1, FR_LDSV + 2, FR_LDSV + 4,
-                              FR_BLKV, FR_V4, FR_V4B, FR_V4L};
-    // A split repeats the flux in every row group: only while the grid is
-    // short of four wavefronts per SIMD (p = 4 pyramids, 34,944 of them: 80
-    // us in two row groups, 98 in one; 196,608: 390 and 359).
-    int last = p->g4;
-    for (int s = 2; s <= p->g4; ++s) {
-        const int gw = flux4_group(p->g4, s*FR_SPLIT + FR_V4L);
-        if (gw == last) continue;
-        if (ncol/64*cdiv(p->g4, last) >= 4096) break;
-        last = gw;
-        cands.push_back(s*FR_SPLIT + FR_V4);
-        cands.push_back(s*FR_SPLIT + FR_V4L);
-    }
-    // the staged form of the smallest split whose operator fits in LDS
-    for (int s = 2; s <= p->g4; ++s)
-        if (flux4_valid(s*FR_SPLIT + FR_V4L, p->g4, p->nc0 + p->nc1)) {
-            cands.push_back(s*FR_SPLIT + FR_V4L);
-            break;
-        }
-    for (int v : cands) {
-        if (is_flux4(v)
-                ? !p->af4 || !flux4_valid(v, p->g4, p->nc0 + p->nc1)
-                : v != FR_BLKV && !variant_valid(v, ldsb, false))
-            continue;
-        FluxPlan q = *p;
-        q.d.variant = v;
-        for (int it = 0; it < reps + 1 && !rc; ++it) {
-            if (it == 1) (void)hipEventRecord(e0, nullptr);
-            rc = flux_launch(&q, 11, ncol, u, ldu, smats, lds, fn, ldf, c,
-                             ncol, rcp, 0, xa, 0, 0, gamma, nullptr);
-        }
-        if (rc) break;
-        (void)hipEventRecord(e1, nullptr);
-        (void)hipEventSynchronize(e1);
-        float ms = 0;
-        (void)hipEventElapsedTime(&ms, e0, e1);
-        if (ms < best) {
-            best = ms;
-            bestv = v;
-        }
-    }
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
-    (void)hipFree(scratch);
-    if (rc) return rc;
-    p->d.variant = bestv;
-    if (variant) *variant = bestv;
-    return 0;
+    return flux_tune(p, false, p->d.variant, ncol, u, ldu, smats, lds, fn,
+                     ldf, gamma, reps, variant);
+    FR_API_END
+}
+
+int frhip_tdivf_plan_tune_rk4(void *plan, int ncol, const void *u, long ldu,
+                              const void *smats, long lds, const void *fn,
+                              long ldf, double gamma, int reps, int *variant)
+{
+    FR_API_BEGIN
+    FluxPlan *p = static_cast<FluxPlan *>(plan);
+    FR_CHECK(p && reps > 0, "invalid arguments");
+    return flux_tune(p, true, p->vrk4, ncol, u, ldu, smats, lds, fn, ldf,
+                     gamma, reps, variant);
     FR_API_END
 }
 
@@ -1855,7 +1905,7 @@ int frhip_tdivf_plan_set_variant(void *plan, int variant)
              variant_valid(variant,
                            (size_t)p->d.mt*(p->d.ks0 + p->d.ks1)*64*esz,
                            false), "invalid variant");
-    p->d.variant = variant;
+    p->d.variant = p->vrk4 = variant;
     return 0;
     FR_API_END
 }
