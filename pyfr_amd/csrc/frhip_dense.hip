@@ -1159,16 +1159,27 @@ int dense_launch(const DensePlan *p, int ep, long ncol, const void *b0,
             return 0;
         }
     }
-    // in place, each column's reads of B must precede its writes: one
-    // wavefront for all rows
-    auto meets = [&](const void *b, int k, long ld) {
-        const uintptr_t b0p = (uintptr_t)b, cp = (uintptr_t)c;
-        return b && b0p < cp + ((p->m - 1)*ldc + ncol)*esz &&
-               cp < b0p + ((k - 1)*ld + ncol)*esz;
+    // Row groups read B in separate blocks, so none may write what another
+    // reads.  Where an output meets an input, one wavefront takes all rows
+    // (its reads precede its writes); past the rows it holds there is no
+    // in-place form, and the scalar kernel serves operands that interleave
+    // without sharing an element, as it did before row groups.
+    const bool acc64 = ep == 3 || ep == 5;
+    auto meets = [&](const void *b, int k, long ld, const void *o,
+                     size_t osz) {
+        const uintptr_t bp = (uintptr_t)b, op = (uintptr_t)o;
+        return b && o && k && bp < op + ((p->m - 1)*ldc + ncol)*osz &&
+               op < bp + ((k - 1)*ld + ncol)*esz;
     };
-    if (variant >= FR_SPLIT && (meets(b0, p->k0, ld0) ||
-                                meets(p->k1 ? b1 : nullptr, p->k1, ld1)))
-        variant %= FR_SPLIT;
+    auto written = [&](const void *b, int k, long ld) {
+        return meets(b, k, ld, c, esz) ||
+               (ep >= 2 && ep <= 5 && meets(b, k, ld, xa, acc64 ? 8 : esz));
+    };
+    if (variant && group_tiles(variant, p->mt) < p->mt &&
+        (written(b0, p->k0, ld0) || written(b1, p->k1, ld1))) {
+        variant = p->mt <= FR_MTMAX ? variant % FR_SPLIT : 0;
+        if (!dense_valid(p, variant)) variant &= ~FR_LDSV;
+    }
     const int rc = p->dtype == FRHIP_F64
         ? launch_t<double>(p, variant, ep, ncol, b0, ld0, b1, ld1, c, ldc,
                            rcp, ldr, nvar, xa, dta, dtb, alpha, beta, s, sl)

@@ -142,6 +142,57 @@ def test_dense_row_groups(backend_factory, precision, variant, shape):
 
 
 @pytest.mark.parametrize('precision', ['double', 'single'])
+@pytest.mark.parametrize('variant', [4, 2*256 + 1, 2*256 + 17, 3*256 + 4])
+@pytest.mark.parametrize('m', [96, 128])
+def test_dense_in_place(backend_factory, precision, variant, m):
+    """C = A B in place, and an RK45 stage whose accumulator is an input,
+    with row groups forced: one wavefront has to take all rows (96 of them,
+    whose operator is staged in LDS by row group only in FP64).  128 rows
+    are more than it holds: as the scalar kernel."""
+    from pyfr_amd.backend import MulProvider
+    be = backend_factory(precision=precision)
+    rng = np.random.default_rng(m)
+    # small entries: in the scalar kernel's order a row's result is an
+    # input of the rows that follow
+    A = 0.03*rng.standard_normal((m, m))
+    v = rng.standard_normal((m, 5, 70))
+    a = be.const_matrix(A)
+    mp = next(p for p in be._providers if isinstance(p, MulProvider))
+    plan = mp._plan(a, be.fpdtype)[0]
+    print(f'\n[in place] {precision} {m} v={variant}', flush=True)
+
+    def mul(var):
+        b = be.matrix((m, 5, 70), v, tags={'align'})
+        be.lib.mul_plan_set_variant(plan, var)
+        be.lib.mul(plan, b.ncol, b.data, b.leaddim, b.data, b.leaddim, 1.0,
+                   0.0, be.stream)
+        be.wait()
+        return b.get()
+    got = mul(variant)
+    if m == 128:
+        assert np.array_equal(got, mul(0))
+        return
+    ref = np.einsum('mk,kvn->mvn', a._host, v)
+    tol = 1e-13 if precision == 'double' else 2e-6
+    assert rel_l2(got, ref) < tol
+
+    A0, A1, b0, b1, c, _ = _operands(be, m, m, 20, 70, 1)
+    rcp = be.matrix((m, 70), 1 + rng.random((m, 70)), tags={'align'})
+    p = _Plan2(be, A0, A1)
+
+    def stage(var):
+        xa = be.matrix((m, 5, 70), b0.get(), tags={'align'})
+        be.lib.mul2_plan_set_variant(p.plan, var)
+        be.lib.mul2(p.plan, c.ncol, xa.data, xa.leaddim, b1.data, b1.leaddim,
+                    c.data, c.leaddim, 2, rcp.data, rcp.leaddim, xa.data,
+                    0.3, -0.7, 0, be.stream)
+        be.wait()
+        return c.get(), xa.get()
+    for x, y in zip(stage(variant), stage(4)):
+        assert np.array_equal(x, y)
+
+
+@pytest.mark.parametrize('precision', ['double', 'single'])
 @pytest.mark.parametrize('variant', [0, 1, 17, 2*256 + 1])
 @pytest.mark.parametrize('m,k,neles', [(40, 20, 70), (18, 10, 1),
                                        (33, 35, 200)])
