@@ -821,10 +821,12 @@ __attribute__((amdgpu_waves_per_eu(G <= 10 ? 4 : 3))) void k_tdivf_flux4(
             float x = invrho*y;
             asm volatile("" : "+v"(x));
             x = v == 0 ? 1.0f : x;
+            // not p times a zero of Sv: an infinite p would reach the density
+            const float pv = v >= 1 && v <= 3 ? p : 0.0f;
 #pragma unroll
             for (int d = 0; d < 3; ++d)
                 b[3*pp + d] = x*(S[d][0]*rv[0] + S[d][1]*rv[1] +
-                                 S[d][2]*rv[2]) + p*Sv[d];
+                                 S[d][2]*rv[2]) + pv*Sv[d];
         }
 #pragma unroll
         for (int k = 0; k < 15; ++k) asm volatile("" : "+v"(b[k]));

@@ -382,6 +382,41 @@ def test_flux4_row_splits(backend_factory, variant):
     test_simplex_rk4_fused_stages(backend_factory, 'single', variant, 4)
 
 
+@pytest.mark.parametrize('variant', [1, 32, 64, 65, 66, 64 + 2*256])
+def test_infinite_pressure_keeps_the_density(backend_factory, variant):
+    """The density flux has no pressure in it: where the pressure of a state
+    is not finite, the momentum and energy of that element are lost, its
+    density is not."""
+    from pyfr_amd.backend import MulProvider
+    be = backend_factory(precision='single', graphs=False)
+    integ, _, _ = _mixed(be, 3, 2, 1, 3)
+    sysm = integ.system
+    rng = np.random.default_rng(5)
+    mp = next(p for p in be._providers if isinstance(p, MulProvider))
+    kerns = {n: e.kernels['tdivf_flux'](0, 1)
+             for n, e in sysm.ele_map.items()}
+    for plan, _, _ in mp._plans3.values():
+        be.lib.tdivf_plan_set_variant(plan, variant)
+    for (n, e), banks in zip(sysm.ele_map.items(), sysm.ele_banks):
+        u = np.ones(banks[0].ioshape) + \
+            0.1*rng.standard_normal(banks[0].ioshape)
+        u[:, 4] += 4
+        e._scal_fpts.set(rng.standard_normal(e._scal_fpts.ioshape))
+        out = []
+        for energy in (5.0, np.inf):
+            u[1, 4, 2] = energy
+            banks[0].set(u)
+            print(f'\n[infinite p] {n} v={variant} E={energy}', flush=True)
+            kerns[n].run(be.stream)
+            be.wait()
+            out.append(banks[1].get())
+        assert np.isfinite(out[0]).all()
+        assert np.array_equal(out[1][:, 0], out[0][:, 0])
+        assert not np.isfinite(out[1][:, 1:, 2]).any()
+        keep = np.arange(u.shape[2]) != 2
+        assert np.array_equal(out[1][..., keep], out[0][..., keep])
+
+
 def test_simplex_rk4_trajectory(backend_factory):
     be = backend_factory()
     integ, orc, u0 = _mixed(be, 3, 2, 1, 3, dt=2e-3)
