@@ -49,8 +49,11 @@ def _warp(x, y, z):
 def _run(make, system, n, order, fuse, scheme=None, steps=2, kind='straight',
          precision='double', **cfgkw):
     be = make(precision=precision, fuse_flux=fuse)
+    consts = cfgkw.pop('constants', {})
     cfg = make_cfg(system, order, precision=precision,
                    scheme=scheme or 'rk4', dt=1e-3, **cfgkw)
+    for k, v in consts.items():
+        cfg.set('constants', k, v)
     kw = {}
     if kind == 'skew':
         kw = {'warp': lambda x, y, z: (x + 0.05*np.sin(y), y, z)}
@@ -139,6 +142,67 @@ def test_ns_rhs(backend_factory, n, order, kind, beta, tau, visc):
     # the viscous terms, a second derivative of fluxes of mu times order 1,
     # stay below the inviscid ones
     assert _rms(got - ref) < _rounding(n, order)
+
+
+# c_p T of the field is about 250
+SUTHERLAND = {'mu': 0.02, 'cpTref': 250.0, 'cpTs': 110.0}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('n,order,kind', [
+    ((5, 4, 3), o, k) for o in (1, 2, 3, 4) for k in ('straight', 'skew')] + [
+    ((6, 6, 6), 2, 'mixed'), ((6, 6, 6), 3, 'mixed')])
+@pytest.mark.parametrize('beta,tau', [(0.0, 0.0), (0.25, 0.1)])
+def test_ns_sutherland(backend_factory, n, order, kind, beta, tau):
+    """Temperature-dependent viscosity, inside the elements and in the
+    normal viscous flux (straight, skew) or the gradients (mixed, p = 1)
+    that the interfaces get."""
+    print(f'\n[hexline sutherland] {n} p={order} {kind} {beta}', flush=True)
+    kw = dict(kind=kind, beta=beta, tau=tau, constants=SUTHERLAND)
+    got, sysm = _run(backend_factory, 'navier-stokes', n, order, True,
+                     visc_corr='sutherland', **kw)
+    assert sysm._nfv == (kind != 'mixed' and order > 1)
+    ref, _ = _run(backend_factory, 'navier-stokes', n, order, False,
+                  visc_corr='sutherland', **kw)
+    assert _rms(got - ref) < _rounding(n, order)
+    plain, _ = _run(backend_factory, 'navier-stokes', n, order, True,
+                    visc_corr='none', **kw)
+    assert _rms(got - plain) > 1e6*_rounding(n, order)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('fuse', [True, False])
+@pytest.mark.parametrize('order', [1, 2, 3])
+def test_sutherland_oracle(backend_factory, fuse, order):
+    """The same against the oracle, in the one-pass kernels and in those
+    they replace."""
+    from oracle.rhs import OracleHexSystem
+    from tests.fr_cases import oracle_consts
+    from tests.test_gpu_parity import rhs_noise_floor
+    print(f'\n[hexline sutherland oracle] p={order} {fuse}', flush=True)
+    got, _ = _run(backend_factory, 'navier-stokes', 3, order, fuse,
+                  visc_corr='sutherland', constants=SUTHERLAND)
+    orc = OracleHexSystem(3, order, 'navier-stokes', constants=oracle_consts(
+        'navier-stokes') | SUTHERLAND | {'visc_corr': 'sutherland'})
+    u0 = orc.ics()
+    err = rel_l2(got, orc.rhs(u0))
+    tol = max(1e-12, 10*rhs_noise_floor(orc, u0))
+    print(f'[hexline sutherland oracle] rel L2 {err:.3e} (tol {tol:.3e})',
+          flush=True)
+    assert err < tol
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('scheme', ['rk4', 'rk45'])
+@pytest.mark.parametrize('order', [1, 2])
+def test_euler_steps_double_whole_blocks(backend_factory, scheme, order):
+    """The stage updates and next-stage traces of the FP64 kernel with 64
+    elements a block, which only grids of 256 blocks and over take."""
+    n = (26, 26, 25)
+    print(f'\n[hexline step 64] p={order} {scheme}', flush=True)
+    got, _ = _run(backend_factory, 'euler', n, order, True, scheme)
+    ref, _ = _run(backend_factory, 'euler', n, order, False, scheme)
+    assert rel_l2(got, ref) < 1e-14
 
 
 @pytest.mark.gpu
