@@ -1625,7 +1625,12 @@ class BaseSystem:
     def max_abs(self, idx):
         return np.max(self._reduce(idx, 'max'), axis=0)
 
+    # how often the host wrote a register: an integrator that keeps a copy
+    # of one (the precision form's FP32 stage input) takes it again
+    host_writes = 0
+
     def set_ele_scal_upts(self, idx, arrs):
+        self.host_writes += 1
         for b, a in zip(self.ele_banks, arrs):
             b[idx].set(a)
 
@@ -1915,11 +1920,13 @@ class MixedRK4Integrator(BaseIntegrator):
             lib.convert(1, w.data, 0, acc.data, acc.nrow*acc.leaddim,
                         be.stream)
         self._work_valid = True
+        self._work_writes = self.system.host_writes
 
     def step(self, t, dt):
         r0, r1 = self.idxcurr, 1 - self.idxcurr
         wa, wb = 2, 3
-        if not self._work_valid:
+        if (not self._work_valid or
+                self._work_writes != self.system.host_writes):
             self._sync_work(r0)
         if self.system.fused_rk4_mixed:
             st = self.system.rhs_rk4_stage
@@ -2017,9 +2024,11 @@ class MixedRK45Integrator(RK45Integrator):
             lib.convert(1, w.data, 0, acc.data, acc.nrow*acc.leaddim,
                         be.stream)
         self._work_valid = True
+        self._work_writes = self.system.host_writes
 
     def step(self, t, dt):
-        if not self._work_valid:
+        if (not self._work_valid or
+                self._work_writes != self.system.host_writes):
             self._sync_work()
         lib, be = self.backend.lib, self.backend
         last = self._nstages - 1

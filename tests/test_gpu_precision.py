@@ -135,3 +135,22 @@ def test_precision_form_euler_rk4(backend_factory):
     errs = field_errors(sols[1], sols[0])
     print(f'\n[precision euler rk4] {errs}', flush=True)
     assert max(errs.values()) < 1e-5, errs
+
+
+@pytest.mark.parametrize('scheme', ['rk4', 'rk45'])
+@pytest.mark.parametrize('fused', [True, False])
+def test_state_set_after_steps(backend_factory, scheme, fused):
+    """A state set after some steps is the one the next step starts from:
+    the FP32 stage input follows it, as in a fresh run."""
+    def run(before, new=None):
+        integ = _integ(backend_factory, 'navier-stokes', 2, 4, 'mixed',
+                       scheme, 1e-3, fused=fused)
+        if new is None:
+            new = integ.soln[0].copy()
+            new[:, 0] *= 1.01
+        integ.run_steps(before)
+        integ.system.set_soln_upts(integ.idxcurr, [new])
+        integ.run_steps(2)
+        return integ.soln[0], new
+    got, state = run(3)
+    assert np.array_equal(got, run(0, state)[0])
