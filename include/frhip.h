@@ -181,9 +181,10 @@ int frhip_hex_plan_create(void **plan, int n, const double *d,
                           const double *ll, const double *lr,
                           const double *x, int dtype);
 int frhip_hex_plan_destroy(void *plan);
-/* geo = FRHIP_GEO_CURVED / FRHIP_GEO_HEX_LINEAR: tdisf (Euler, pyfr/solvers/
- * euler/kernels/tflux.mako:8-30) + tdivtpcorf + tdivtconf + negdivconf of
- * the solution u (n^3, 5, neles); gm: smats or vertices.  geo = -1: u holds
+/* geo = FRHIP_GEO_CURVED / FRHIP_GEO_HEX_LINEAR (n > 2): tdisf (Euler,
+ * pyfr/solvers/euler/kernels/tflux.mako:8-30) + tdivtpcorf + tdivtconf +
+ * negdivconf of the solution u (n^3, 5, neles); gm: smats or vertices.
+ * geo = -1: u holds
  * the volume part of the transformed divergence (frhip_hex_nsvol) and
  * tdivtconf + negdivconf are applied.  f (6 n^2, 5, neles): the common
  * normal fluxes.  ep (1-3, 10-17), c, rcp (a value per point), xa, dta, dtb

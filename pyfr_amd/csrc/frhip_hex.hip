@@ -878,10 +878,11 @@ template <typename T, int N>
 static int hex_div_n(const HexPlan *p, int geo, const HexDivArgs<T> &a,
                      hipStream_t s)
 {
+    if constexpr (N > 2)
+        if (geo == FRHIP_GEO_HEX_LINEAR)
+            return hex_div_launch<T, N, FRHIP_GEO_HEX_LINEAR>(p, a, s);
     return geo < 0 ? hex_div_launch<T, N, -1>(p, a, s)
-         : geo == FRHIP_GEO_HEX_LINEAR
-               ? hex_div_launch<T, N, FRHIP_GEO_HEX_LINEAR>(p, a, s)
-               : hex_div_launch<T, N, FRHIP_GEO_CURVED>(p, a, s);
+                   : hex_div_launch<T, N, FRHIP_GEO_CURVED>(p, a, s);
 }
 
 template <typename T>
@@ -921,10 +922,11 @@ static int hex_ns_n(const HexPlan *p, int geo, const HexNsArgs<T> &a,
     constexpr int EB = hex_ns_eb<T, N>();
     const dim3 grid(cdiv(a.neles, EB)), block(N*N*N*EB);
     const auto *line = static_cast<const HexLine<T, N> *>(p->line);
-    auto k = a.fn ? k_hex_nsvol<T, N, FRHIP_GEO_HEX_LINEAR, true, EB>
-           : geo == FRHIP_GEO_HEX_LINEAR
-               ? k_hex_nsvol<T, N, FRHIP_GEO_HEX_LINEAR, false, EB>
-               : k_hex_nsvol<T, N, FRHIP_GEO_CURVED, false, EB>;
+    auto k = k_hex_nsvol<T, N, FRHIP_GEO_CURVED, false, EB>;
+    if constexpr (N > 2)
+        if (geo == FRHIP_GEO_HEX_LINEAR)
+            k = a.fn ? k_hex_nsvol<T, N, FRHIP_GEO_HEX_LINEAR, true, EB>
+                     : k_hex_nsvol<T, N, FRHIP_GEO_HEX_LINEAR, false, EB>;
     hipLaunchKernelGGL(k, grid, block, 0, s, line, a);
     FR_LAUNCHED();
     return 0;
@@ -1006,7 +1008,9 @@ int frhip_hex_div(void *plan, int geo, int neles, const void *u, long ldu,
     FR_API_BEGIN
     HexPlan *p = static_cast<HexPlan *>(plan);
     FR_CHECK(p && u && f && c && rcp, "null argument");
-    FR_CHECK(geo >= -1 && geo <= 1 && (geo < 0 || gm),
+    // p = 1 hexes take their stored metric, as in the reference (pyfr/
+    // solvers/base/elements.py:224-227)
+    FR_CHECK(geo >= -1 && geo <= (p->n > 2) && (geo < 0 || gm),
              "invalid geometry mode");
     FR_CHECK((ep >= 1 && ep <= 3) || (ep >= 10 && ep <= 17),
              "invalid epilogue");
@@ -1046,7 +1050,7 @@ int frhip_hex_nsvol(void *plan, int geo, int neles, const void *u, long ldu,
     FR_API_BEGIN
     HexPlan *p = static_cast<HexPlan *>(plan);
     FR_CHECK(p && u && cm && gm && dv && g && consts, "null argument");
-    FR_CHECK(geo == FRHIP_GEO_HEX_LINEAR ||
+    FR_CHECK((geo == FRHIP_GEO_HEX_LINEAR && p->n > 2) ||
              (geo == FRHIP_GEO_CURVED && rcp && !fn),
              "invalid geometry mode");
     FR_CHECK(neles >= 0, "invalid extents");
