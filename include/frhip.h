@@ -205,16 +205,17 @@ int frhip_hex_div(void *plan, int geo, int neles, const void *u, long ldu,
  * whole blocks of 64 elements); dv
  * (n^3, 5, neles) receives the volume part of the transformed divergence
  * and g the physical gradients at the flux points (3, 6 n^2, 5, neles),
- * which may hold cm in its first 6 n^2 rows, or, with fn (linear hexes),
+ * which may hold cm in its first 6 n^2 rows, or, with nfv (linear hexes),
  * (6 n^2, 5, neles): the viscous flux along the element's own unnormalised
- * outward normal (variable 0, which has none, is not written).  fn (18, 3,
- * neles), leading dimension ldg: for face f that normal is row 3f + x row
- * 3f + 1 + y row 3f + 2 at its coordinates (x, y).  consts and base: as
+ * outward normal (variable 0, which has none, is not written).  FP64 forms
+ * that normal from the vertices; FP32 reads fn (18, 3, neles), leading
+ * dimension ldg: for face f, row 3f + x row 3f + 1 + y row 3f + 2 at its
+ * coordinates (x, y).  consts and base: as
  * frhip_tflux_ns. */
 int frhip_hex_nsvol(void *plan, int geo, int neles, const void *u, long ldu,
                     const void *cm, long ldcm, const void *gm, long ldg,
                     const void *rcp, long ldr, void *dv, long ldd, void *g,
-                    long ldgr, const void *fn, const double *consts,
+                    long ldgr, int nfv, const void *fn, const double *consts,
                     const double *base, void *stream);
 
 /* ---- flux-fused divergence for straight-sided tets and prisms (Euler):
@@ -362,7 +363,7 @@ int frhip_intcflux_ns(int dtype, int rsolver, int n, void *ubase,
                       const void *nl, long ldn, const double *consts,
                       double pmin, const void *mu_p, const double *bstate,
                       void *stream);
-/* The same from each side's normal viscous flux (frhip_hex_nsvol, fn) at
+/* The same from each side's normal viscous flux (frhip_hex_nsvol, nfv) at
  * vbase + lmap[i], vbase + rmap[i]; the two sides' normals must be opposite
  * to rounding. */
 int frhip_intcflux_nfv(int dtype, int rsolver, int n, void *ubase,

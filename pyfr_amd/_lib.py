@@ -91,7 +91,7 @@ _FUNCS = {
     'frhip_intcflux_nfv': [_I, _I, _I, _P, _PI32, _PI32, _P, _P, _L, _P, _D,
                            _P, _P],
     'frhip_hex_nsvol': [_P, _I, _I, _P, _L, _P, _L, _P, _L, _P, _L, _P, _L,
-                        _P, _L, _P, _P, _P, _P],
+                        _P, _L, _I, _P, _P, _P, _P],
     'frhip_bccflux_euler': [_I, _I, _I, _I, _P, _PI32, _P, _L, _P, _L, _P,
                             _D, _P],
     'frhip_bcconu': [_I, _I, _I, _P, _PI32, _P, _PI32, _P, _L, _P, _L, _P,

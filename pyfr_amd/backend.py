@@ -943,12 +943,12 @@ class HexLineProvider:
         return k
 
     def hexns(self, basis, geo, neles, u, comm, dv, grad, tplargs, metric,
-              rcpdjac, fnorms=None):
+              rcpdjac, nfv=False, fnorms=None):
         """tgradpcoru + tgradcoru + tdisf + tdivtpcorf + gradcoru_fpts over
         neles elements: dv's first nupts rows receive the volume divergence,
-        grad the gradients at the flux points or (fnorms: the faces' normals,
-        ``linear_hex_face_normals``) its second nfpts rows each side's
-        normal viscous flux."""
+        grad the gradients at the flux points or (nfv) its second nfpts rows
+        each side's normal viscous flux, in FP32 along fnorms
+        (``linear_hex_face_normals``)."""
         nu, nf = basis.nupts, basis.nfpts
         if (u.nrow != nu or comm.nrow < nf or dv.nrow < nu or
                 grad.nrow != 3*nf or any(m.ncol != u.ncol or
@@ -959,15 +959,14 @@ class HexLineProvider:
                  (fnorms.nrow != 18 or fnorms.dtype != u.dtype or
                   fnorms.leaddim != metric.leaddim))):
             raise ValueError('Incompatible matrices for hexns')
-        nfv = fnorms is not None
         plan = self._plan(basis, u.dtype)
         base = PointwiseProvider._base(tplargs)
         consts = PointwiseProvider._ns_consts(tplargs)
         gp = grad.data + (nf*grad.leaddim*grad.itemsize if nfv else 0)
         args = (plan, geo, neles, u.data, u.leaddim, comm.data, comm.leaddim,
                 metric.data, metric.leaddim, rcpdjac.data, rcpdjac.leaddim,
-                dv.data, dv.leaddim, gp, grad.leaddim,
-                fnorms.data if nfv else None, consts, base)
+                dv.data, dv.leaddim, gp, grad.leaddim, int(nfv),
+                None if fnorms is None else fnorms.data, consts, base)
         lib = self.backend.lib
         return Kernel(lambda stream: lib.hex_nsvol(*args, stream),
                       mats=(u, comm, dv, grad, metric, fnorms),

@@ -519,7 +519,7 @@ struct HexNsArgs {
     long ldg;
     const T *rcp;
     long ldr;
-    const T *fn;        // NFV: the faces' normals, rows of ldg
+    const T *fn;        // NFV in FP32: the faces' normals, rows of ldg
     T *dv;              // volume part of the transformed divergence
     long ldd;
     T *g;               // gradients (3, nfpts, 5, E) or normal viscous flux
@@ -606,10 +606,13 @@ struct HexFace {
 // LDS buffer; all of the (3, Nu, 5) and (3, Nf, 5) intermediates of the
 // kernels replaced stay in registers and LDS.  NFV: at the flux points only
 // the normal viscous flux of this side (4 values) instead of the gradients
-// (15), for meshes whose interface kernel needs no more.  The normal comes
-// from coefficients formed in FP64 and rounded once: rebuilt from FP32
+// (15), for meshes whose interface kernel needs no more.  In FP32 the normal
+// comes from coefficients formed in FP64 and rounded once: rebuilt from FP32
 // vertices it was off by 4e-6 of its length on 48^3 elements of [0, 2 pi],
-// 8e-5 with the box at 100.
+// 8e-5 with the box at 100 (48^3 p = 3 steps of the precision form 3.97
+// against 4.03 ms: 54 values an element).  FP64 vertices lose nothing, and
+// the coefficients cost 3 % of the kernel (64^3 p = 3: 1,271 against 1,307
+// us).
 template <typename T, int N, int GEO, bool NFV, int EB>
 __global__ __launch_bounds__(N*N*N*EB)
 __attribute__((amdgpu_waves_per_eu(4))) void k_hex_nsvol(
@@ -733,16 +736,42 @@ __attribute__((amdgpu_waves_per_eu(4))) void k_hex_nsvol(
         const HexFace h = HexFace::of<N>(q);
         int p0, st;
         h.line<N>(p0, st);
-        // this side's normal (linear in each of the face's coordinates: their
-        // product's coefficient vanishes) and its state
+        // this side's normal and state
         T nf[3] = {}, uf[5] = {};
         if constexpr (NFV) {
             const T x = line->x[h.a], y = line->x[h.b];
-            const T *gn = a.fn + 3*(q/NN)*a.ldg + soa_ix(e, 0, 3);
+            if constexpr (sizeof(T) == 4) {
+                // linear in each of the face's coordinates: their product's
+                // coefficient vanishes
+                const T *gn = a.fn + 3*(q/NN)*a.ldg + soa_ix(e, 0, 3);
 #pragma unroll
-            for (int b = 0; b < 3; ++b)
-                nf[b] = fma(y, gn[2*a.ldg + b*SOA],
-                            fma(x, gn[a.ldg + b*SOA], gn[b*SOA]));
+                for (int b = 0; b < 3; ++b)
+                    nf[b] = fma(y, gn[2*a.ldg + b*SOA],
+                                fma(x, gn[a.ldg + b*SOA], gn[b*SOA]));
+            }
+            else {
+                // the tangents along the face's axes, from its four vertices
+                T ts[3], tt[3];
+                const int sa = h.axis == 0 ? 1 : 0, ta = h.axis == 2 ? 1 : 2;
+                const int v0 = h.side << h.axis;
+                const T *gv = a.geo + soa_ix(e, 0, 3);
+#pragma unroll
+                for (int b = 0; b < 3; ++b) {
+                    const T w00 = gv[v0*a.ldg + b*SOA];
+                    const T w10 = gv[(v0 | 1 << sa)*a.ldg + b*SOA];
+                    const T w01 = gv[(v0 | 1 << ta)*a.ldg + b*SOA];
+                    const T w11 = gv[(v0 | 1 << sa | 1 << ta)*a.ldg + b*SOA];
+                    ts[b] = T(0.25)*((T(1) - y)*(w10 - w00) +
+                                     (T(1) + y)*(w11 - w01));
+                    tt[b] = T(0.25)*((T(1) - x)*(w01 - w00) +
+                                     (T(1) + x)*(w11 - w10));
+                }
+                PencilGeo<T>::cross(ts, tt, nf);
+                // axes (y, z), (x, z), (x, y): the middle one is left-handed
+                const T sg = (h.axis == 1) != (h.side == 0) ? T(-1) : T(1);
+#pragma unroll
+                for (int b = 0; b < 3; ++b) nf[b] *= sg;
+            }
             layer_end(nf);
 #pragma unroll
             for (int m = 0; m < N; ++m) {
@@ -916,7 +945,7 @@ constexpr int hex_ns_eb()
 }
 
 template <typename T, int N>
-static int hex_ns_n(const HexPlan *p, int geo, const HexNsArgs<T> &a,
+static int hex_ns_n(const HexPlan *p, int geo, int nfv, const HexNsArgs<T> &a,
                     hipStream_t s)
 {
     constexpr int EB = hex_ns_eb<T, N>();
@@ -925,18 +954,18 @@ static int hex_ns_n(const HexPlan *p, int geo, const HexNsArgs<T> &a,
     auto k = k_hex_nsvol<T, N, FRHIP_GEO_CURVED, false, EB>;
     if constexpr (N > 2)
         if (geo == FRHIP_GEO_HEX_LINEAR)
-            k = a.fn ? k_hex_nsvol<T, N, FRHIP_GEO_HEX_LINEAR, true, EB>
-                     : k_hex_nsvol<T, N, FRHIP_GEO_HEX_LINEAR, false, EB>;
+            k = nfv ? k_hex_nsvol<T, N, FRHIP_GEO_HEX_LINEAR, true, EB>
+                    : k_hex_nsvol<T, N, FRHIP_GEO_HEX_LINEAR, false, EB>;
     hipLaunchKernelGGL(k, grid, block, 0, s, line, a);
     FR_LAUNCHED();
     return 0;
 }
 
 template <typename T>
-static int hex_ns_t(const HexPlan *p, int geo, const void *fn, int neles,
+static int hex_ns_t(const HexPlan *p, int geo, int nfv, int neles,
                     const void *u, long ldu, const void *cm, long ldcm,
                     const void *gm, long ldg, const void *rcp, long ldr,
-                    void *dv, long ldd, void *g, long ldgr,
+                    void *dv, long ldd, void *g, long ldgr, const void *fn,
                     const double *consts, const double *base, hipStream_t s)
 {
     const HexNsArgs<T> a{neles, (const T *)u, ldu, (const T *)cm, ldcm,
@@ -946,10 +975,10 @@ static int hex_ns_t(const HexPlan *p, int geo, const void *fn, int neles,
                          base ? base_state<T>(base, consts[0])
                               : BaseState<T>{}};
     switch (p->n) {
-        case 2: return hex_ns_n<T, 2>(p, geo, a, s);
-        case 3: return hex_ns_n<T, 3>(p, geo, a, s);
-        case 4: return hex_ns_n<T, 4>(p, geo, a, s);
-        default: return hex_ns_n<T, 5>(p, geo, a, s);
+        case 2: return hex_ns_n<T, 2>(p, geo, nfv, a, s);
+        case 3: return hex_ns_n<T, 3>(p, geo, nfv, a, s);
+        case 4: return hex_ns_n<T, 4>(p, geo, nfv, a, s);
+        default: return hex_ns_n<T, 5>(p, geo, nfv, a, s);
     }
 }
 
@@ -1044,15 +1073,17 @@ int frhip_hex_div(void *plan, int geo, int neles, const void *u, long ldu,
 int frhip_hex_nsvol(void *plan, int geo, int neles, const void *u, long ldu,
                     const void *cm, long ldcm, const void *gm, long ldg,
                     const void *rcp, long ldr, void *dv, long ldd, void *g,
-                    long ldgr, const void *fn, const double *consts,
+                    long ldgr, int nfv, const void *fn, const double *consts,
                     const double *base, void *stream)
 {
     FR_API_BEGIN
     HexPlan *p = static_cast<HexPlan *>(plan);
     FR_CHECK(p && u && cm && gm && dv && g && consts, "null argument");
     FR_CHECK((geo == FRHIP_GEO_HEX_LINEAR && p->n > 2) ||
-             (geo == FRHIP_GEO_CURVED && rcp && !fn),
+             (geo == FRHIP_GEO_CURVED && rcp && !nfv),
              "invalid geometry mode");
+    FR_CHECK(!nfv || fn || p->dtype == FRHIP_F64,
+             "normal viscous fluxes in FP32 need the faces' normals");
     FR_CHECK(neles >= 0, "invalid extents");
     const long ncol = 320L*((neles + 63L)/64);
     FR_CHECK(ldu >= ncol && ldcm >= ncol && ldd >= ncol && ldgr >= ncol &&
@@ -1063,10 +1094,10 @@ int frhip_hex_nsvol(void *plan, int geo, int neles, const void *u, long ldu,
     if (neles == 0) return 0;
     hipStream_t s = as_stream(stream);
     return p->dtype == FRHIP_F64
-        ? hex_ns_t<double>(p, geo, fn, neles, u, ldu, cm, ldcm, gm, ldg, rcp,
-                           ldr, dv, ldd, g, ldgr, consts, base, s)
-        : hex_ns_t<float>(p, geo, fn, neles, u, ldu, cm, ldcm, gm, ldg, rcp,
-                          ldr, dv, ldd, g, ldgr, consts, base, s);
+        ? hex_ns_t<double>(p, geo, nfv, neles, u, ldu, cm, ldcm, gm, ldg, rcp,
+                           ldr, dv, ldd, g, ldgr, fn, consts, base, s)
+        : hex_ns_t<float>(p, geo, nfv, neles, u, ldu, cm, ldcm, gm, ldg, rcp,
+                          ldr, dv, ldd, g, ldgr, fn, consts, base, s);
     FR_API_END
 }
 

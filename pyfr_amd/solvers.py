@@ -765,8 +765,9 @@ class NavierStokesElements(EulerElements):
                     'hexns', self.basis, mode, n, s(self.scal_upts[uin]),
                     s(self._vect_fpts), s(self._vect_upts),
                     s(self._vect_fpts), tplargs | self.base_tpl, metric,
-                    s(self._rcpdjac_upts),
-                    fnorms=self._fnorms_linear if nfv else None))
+                    s(self._rcpdjac_upts), nfv=nfv,
+                    fnorms=self._fnorms_linear
+                    if nfv and be.fpdtype == np.float32 else None))
 
             def hexdiv(fout, xa=None, stage=None, disu=False):
                 return be.kernel(

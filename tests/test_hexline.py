@@ -328,7 +328,7 @@ def test_short_metric_rows_are_refused(backend_factory, precision, order,
     def ns(ldr):
         be.lib.hex_nsvol(plan, 0, neles, u.data, u.leaddim, f.data,
                          f.leaddim, s.data, s.leaddim, r.data, ldr, c.data,
-                         c.leaddim, g.data, g.leaddim, 0, consts, None,
+                         c.leaddim, g.data, g.leaddim, 0, None, consts, None,
                          be.stream)
     print(f'\n[hexline ldr] {precision} p={order} {neles}', flush=True)
     for call in (div, ns):
@@ -338,6 +338,13 @@ def test_short_metric_rows_are_refused(backend_factory, precision, order,
         call(r.leaddim)
     be.wait()
     assert np.isfinite(c.get()).all() and np.isfinite(g.get()).all()
+    if precision == 'single':
+        # the normal viscous flux in FP32 takes the faces' normals
+        with pytest.raises(FrHipError, match='normals'):
+            be.lib.hex_nsvol(plan, 1, neles, u.data, u.leaddim, f.data,
+                             f.leaddim, s.data, s.leaddim, None, 0, c.data,
+                             c.leaddim, g.data, g.leaddim, 1, None, consts,
+                             None, be.stream)
 
 
 @pytest.mark.parametrize('order,neles', [(2, 1), (4, 100)])
