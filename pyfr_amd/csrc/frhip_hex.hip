@@ -50,10 +50,13 @@ constexpr int hex_eb()
 }
 
 // A grid that leaves CUs without a block takes 16-element blocks (8^3 p = 2:
-// 86 against 109 us a step).
-static int hex_eb_for(int eb, int neles)
+// 86 against 109 us a step), but not at p = 1 in FP32: such a block is one
+// wavefront, whose rows are half a line (RK4 steps with 64 / 16 elements,
+// 11^3: 69 / 80 us, 28^3: 107 / 131; in FP64 14^3: 76 / 72).
+template <typename T, int N>
+constexpr int hex_eb_short()
 {
-    return cdiv(neles, eb) < 256 ? 16 : eb;
+    return N > 2 || sizeof(T) == 8 ? 16 : hex_eb<T, N>();
 }
 
 // 1-D operators, on the device: d[i][m] the derivative corrected for the
@@ -879,14 +882,14 @@ template <typename T, int N, int GEO>
 static int hex_div_launch(const HexPlan *p, const HexDivArgs<T> &a,
                           hipStream_t s)
 {
-    constexpr int EB = hex_eb<T, N>();
-    const int eb = hex_eb_for(EB, a.neles);
+    constexpr int EB = hex_eb<T, N>(), EBS = hex_eb_short<T, N>();
+    const int eb = cdiv(a.neles, EB) < 256 ? EBS : EB;
     const dim3 grid(cdiv(a.neles, eb)), block(N*N*eb);
     const auto *line = static_cast<const HexLine<T, N> *>(p->line);
 #define FR_FAM(F)                                                           \
     case F: {                                                               \
         auto k = eb == EB ? k_hex_div<T, N, GEO, F, EB>                     \
-                          : k_hex_div<T, N, GEO, F, 16>;                    \
+                          : k_hex_div<T, N, GEO, F, EBS>;                   \
         hipLaunchKernelGGL(k, grid, block, 0, s, line, a);                  \
         break;                                                              \
     }
